@@ -114,9 +114,11 @@ typedef struct slm_config {
  * floor and deposit cell are taken in f64.  Agents are still exchanged as f32. */
 #define SLM_FLAG_F64_POSITIONS 0x2u
 /* With re-sorting on, stage each 64x64-cell tile's trail window (tile plus
- * sensor reach plus drift since the re-sort) in LDS and sense from there; taps
- * outside the window read global memory, so results are unchanged.  Pays off
- * for short sensor distances and frequent re-sorts. */
+ * sensor reach plus drift since the re-sort) in LDS and sense from there; agents
+ * that the window does not cover, and tiles whose window does not fit 80 KiB, read
+ * global memory, so results are unchanged.  Without the flag the library does so
+ * by itself where it pays (from 2^21 agents on, one agent to four cells, windows
+ * that fit); with it, wherever there is a re-sort. */
 #define SLM_FLAG_TILED_SENSING 0x4u
 /* With BF16 storage: the trail pass stores each cell rounded up with
  * probability equal to the discarded fraction of its f32 value, instead of to
@@ -200,7 +202,10 @@ int slm_destroy(slm_sim* sim);
 /* Replace the parameters for subsequent steps; agents and trail persist.
  * Replaces update_settings / the preset switch (src/main.rs:83-99, :815-832).
  * Captured graphs stay valid: kernels read parameters from device memory.
- * One exception, with SLM_FLAG_GAUSSIAN_DIFFUSE: a 16-bit pool's Gaussian pass
+ * Two exceptions.  Where the library senses through tile windows (see
+ * SLM_FLAG_TILED_SENSING), a change of sensor distance or speeds that changes how
+ * many steps after a re-sort the windows fit drops the captured graphs likewise.
+ * And with SLM_FLAG_GAUSSIAN_DIFFUSE: a 16-bit pool's Gaussian pass
  * sizes its LDS tile (and its tile height) for the largest radius class
  * (R <= 2, <= 4, <= 8) of its instances, so a change of class waits for the
  * handle's stream, drops the captured graphs (the next slm_step recaptures
@@ -323,7 +328,8 @@ typedef struct slm_tuning {
                                 columns): 4, 8, 16, 32 or 64; 0 = chosen from the
                                 grid so the launch has >= 8192 waves */
   uint32_t tiled_sensing;    /* 1 = SLM_FLAG_TILED_SENSING (needs re-sorting),
-                                2 = SLM_FLAG_WINDOW_SENSING, 0 = neither */
+                                2 = SLM_FLAG_WINDOW_SENSING, 0 = the library's
+                                choice of global memory or tile windows */
   uint32_t trials;           /* autotune: configurations timed; else 0 */
   uint32_t instance_groups;  /* 1..4096 (0 reads as 1): between re-sorts the
                                 instances step as this many contiguous groups

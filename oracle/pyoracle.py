@@ -33,6 +33,8 @@ def lib():
         L = ctypes.CDLL(LIB_PATH)
         sig = {
             "orc_sincos": (None, [ctypes.c_float, _F, _F]),
+            "orc_trig_small_mismatches": (ctypes.c_uint64, [ctypes.c_uint32] * 3),
+            "orc_trig_mid_mismatches": (ctypes.c_uint64, [ctypes.c_uint32] * 3),
             "orc_set_libm_trig": (None, [ctypes.c_int]),
             "orc_wgsl_mod": (ctypes.c_float, [ctypes.c_float, ctypes.c_float]),
             "orc_fract": (ctypes.c_float, [ctypes.c_float]),

@@ -24,6 +24,30 @@
 
 void orc_sincos(float x, float* s, float* c) { slm_sincosf(x, s, c); }
 
+/* How many of the floats +-x, x's bits lo, lo + step, ... below hi, the short forms
+ * of slm_trig.h give other bits for than the general one. */
+uint64_t orc_trig_small_mismatches(uint32_t lo, uint32_t hi, uint32_t step) {
+  uint64_t bad = 0;
+  for (uint64_t u = lo; u < hi; u += step)
+    for (int neg = 0; neg < 2; neg++) {
+      float x = slm_f32_from_bits((uint32_t)u | (neg ? 0x80000000u : 0u)), s, c, s2, c2;
+      slm_sincosf_finite(x, &s, &c);
+      slm_sincosf_small(x, &s2, &c2);
+      bad += slm_f32_bits(s) != slm_f32_bits(s2) || slm_f32_bits(c) != slm_f32_bits(c2);
+    }
+  return bad;
+}
+uint64_t orc_trig_mid_mismatches(uint32_t lo, uint32_t hi, uint32_t step) {
+  uint64_t bad = 0;
+  for (uint64_t u = lo; u < hi; u += step)
+    for (int neg = 0; neg < 2; neg++) {
+      float x = slm_f32_from_bits((uint32_t)u | (neg ? 0x80000000u : 0u)), s, c;
+      slm_sincosf_finite(x, &s, &c);
+      bad += slm_f32_bits(s) != slm_f32_bits(slm_sinf_mid(x));
+    }
+  return bad;
+}
+
 /* The agent update's sin/cos: the shared implementation, or (for tests that
  * model a reference whose transcendental bits differ) the C library's. */
 static int g_libm_trig = 0;

@@ -54,6 +54,8 @@ enum { ORC_STORAGE_F32 = 0, ORC_STORAGE_BF16 = 1, ORC_STORAGE_F16 = 2, ORC_STORA
 
 /* ---- primitives (exposed for the known-answer tests) -------------------- */
 void orc_sincos(float x, float* s, float* c);
+uint64_t orc_trig_small_mismatches(uint32_t lo, uint32_t hi, uint32_t step);
+uint64_t orc_trig_mid_mismatches(uint32_t lo, uint32_t hi, uint32_t step);
 /* Switch the agent update between the shared sin/cos (default, 0) and the C
  * library's sinf/cosf (1): a stand-in for a reference whose transcendental
  * bits differ, for statistical (not bitwise) comparisons. */

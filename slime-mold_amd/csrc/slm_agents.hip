@@ -82,6 +82,11 @@ struct TrailRead<SLM_STORAGE_BF16> {
     a = __uint_as_float((w & 0x7fffu) << 16);
     b = __uint_as_float(((w >> 16) & 0x7fffu) << 16);
   }
+  // |T| of the two cells in a word.
+  __device__ static void split(uint32_t w, float& a, float& b) {
+    a = __builtin_fabsf(__uint_as_float(w << 16));
+    b = __uint_as_float(w & 0x7fff0000u);
+  }
   __device__ static void mark(void* t, uint32_t i) { mark16(t, i); }
 };
 
@@ -93,7 +98,9 @@ struct TrailRead<SLM_STORAGE_F16> {
     return static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(raw)));
   }
   __device__ static void load_pair(const void* t, uint32_t i, float& a, float& b) {
-    uint32_t w = load_u16_pair(t, i);
+    split(load_u16_pair(t, i), a, b);
+  }
+  __device__ static void split(uint32_t w, float& a, float& b) {
     a = static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(w & 0x7fffu)));
     b = static_cast<float>(
         __builtin_bit_cast(_Float16, static_cast<uint16_t>((w >> 16) & 0x7fffu)));
@@ -166,50 +173,6 @@ struct GlobalTaps {
     return sample_at<S>(t, w, h, x0, y0, dx, dy);
   }
   __device__ void mark(uint32_t x, uint32_t y) const { TrailRead<S>::mark(t, __umul24(y, w) + x); }
-};
-
-// Taps from a window of the trail staged in LDS (|T| values of cells
-// [wx0, wx0+ww) x [wy0, wy0+wh)); taps outside it go to global memory, so
-// the result does not depend on the window.
-template <int S>
-struct WindowTaps {
-  using elem = typename TrailRead<S>::elem;
-  void* t;
-  uint32_t w, h;
-  const elem* win;
-  int wx0, wy0, ww, wh;
-  __device__ float sample(int x0, int y0, float dx, float dy) const {
-    bool in = x0 >= 0 && static_cast<uint32_t>(x0) < w - 1u && y0 >= 0 &&
-              static_cast<uint32_t>(y0) < h - 1u;
-    int lx = x0 - wx0, ly = y0 - wy0;
-    bool inw = in && lx >= 0 && lx + 1 < ww && ly >= 0 && ly + 1 < wh;
-    float v00, v10, v01, v11;
-    if (inw) {
-      int i = ly * ww + lx;
-      v00 = TrailRead<S>::value(win[i]);
-      v10 = TrailRead<S>::value(win[i + 1]);
-      v01 = TrailRead<S>::value(win[i + ww]);
-      v11 = TrailRead<S>::value(win[i + ww + 1]);
-    } else {
-      uint32_t i00 = in ? __umul24(static_cast<uint32_t>(y0), w) + static_cast<uint32_t>(x0) : 0u;
-      uint32_t down = in ? w : 0u;
-      TrailRead<S>::load_pair(t, i00, v00, v10);
-      TrailRead<S>::load_pair(t, i00 + down, v01, v11);
-    }
-    float v0 = wgsl_mix(v00, v10, dx);
-    float v1 = wgsl_mix(v01, v11, dx);
-    float v = wgsl_mix(v0, v1, dy);
-    return in ? v : 0.0f;
-  }
-  // Inside the window |T| is known, so the mark is a store only.
-  __device__ void mark(uint32_t x, uint32_t y) const {
-    int lx = static_cast<int>(x) - wx0, ly = static_cast<int>(y) - wy0;
-    if (lx >= 0 && lx < ww && ly >= 0 && ly < wh)
-      static_cast<elem*>(t)[__umul24(y, w) + x] =
-          static_cast<elem>(static_cast<uint32_t>(win[ly * ww + lx]) | TrailRead<S>::kSign);
-    else
-      TrailRead<S>::mark(t, __umul24(y, w) + x);
-  }
 };
 
 // Taps from a workgroup's window of the trail staged in LDS (windowed
@@ -670,23 +633,388 @@ __global__ __launch_bounds__(kAgentBlock) void agents_kernel(
   });
 }
 
-// ---- tiled sensing -----------------------------------------------------------
+// ---- tile windows ------------------------------------------------------------
 // After a re-sort the agents of each 2^k x 2^k-cell tile occupy consecutive
 // slots (the tile is an aligned square of Morton bins).  One workgroup takes a
-// work item (a tile's slots, at most kItemAgents) and stages the trail around
-// the tile - the tile plus a margin covering the sensor distance and the
-// distance agents may have drifted since the re-sort - in LDS once, so sensing
-// reads LDS instead of issuing divergent global loads (which kept the texture
-// address unit ~97% busy).  Taps that still fall outside use global memory.
-constexpr int kTiledBlock = 1024;
+// work item (up to 1.5 * kItemAgents of a tile's slots) and stages the trail
+// around the tile - the tile plus a margin of the sensor reach and the distance
+// agents may have drifted since the re-sort - in LDS, as f32, and senses there.
+//
+// Why: the vector L1 serves a divergent gather one lane a cycle whatever lines
+// the lanes share: a wave of 64 agents costs the global pass 525 accesses (384
+// of them the six tap pairs, 128 the mark's load and store), which at 2.35 GHz
+// are exactly its 229 us on 4096^2 with 2^24 agents once trails have formed.
+// The LDS reads the same pairs at 64 banks a cycle, and the window comes in
+// coalesced, 16 bytes a lane: 4.4 cells an agent at one agent a cell.  What it
+// measured, us per pass with the global pass's in brackets: 4096^2 f32 with 2^24
+// agents 180 (275) while trails form, 159 (205) once formed; 1600 x 900 with
+// 10^7 agents 96 (137) and 78 (109); 8192^2 bf16 with f64 positions and 2^26
+// agents 890 to 915 (1030 to 1200).
+//
+// Shape, all measured: 64-cell tiles and 1024 threads, two workgroups to a CU
+// (80 KiB of LDS each, 64 VGPRs), so that one computes while the other stages;
+// 32-cell tiles with 512 threads are 25% slower (they stage twice the cells),
+// a persistent workgroup holding the next window in registers 15% slower (half
+// the waves).  f64 positions need more registers: 512 threads.
+//
+// An agent's wave senses from the window when all its agents are where the
+// margin covers them (a test per agent, so results never depend on the margin,
+// the work list or the time since the re-sort) and angles and parameters are in
+// the ordinary range, else it takes agent_update and reads global memory.
+//
+// The update itself is then bound by VALU issue.  On gfx950 f32 multiply, add
+// and fma, and/xor/bitop3, right shifts and 32-bit adds issue in 2.3 cycles per
+// wave when every operand is a vector register or a literal; with a scalar
+// register operand, and for compares, selects, conversions, rounding, left
+// shifts and 64-bit address adds, it is 4.4 (measured).  So tile_update keeps its
+// uniform operands in vector registers (in_vgpr), replaces selects by bit
+// operations and skips the range tests where the window is not clipped by the
+// grid's edge: 239 instead of 325 VALU instructions per wave.  (The global pass
+// keeps its own form: it gains nothing from fewer instructions.)
+// A cell's mark in two halves, the load of the 16 bits that hold its sign and
+// their store, so that a caller can have other stores between them.
+struct Mark {
+  uint16_t* p;
+  uint32_t raw;
+  __device__ void store() const { *p = static_cast<uint16_t>(raw | 0x8000u); }
+};
 
-// Largest square window of `elem_bytes` cells that fits kWindowBytes.
-constexpr int window_side_of(size_t elem_bytes) {
-  int side = 1;
-  while (static_cast<size_t>(side + 1) * (side + 1) * elem_bytes <= kWindowBytes) side++;
-  return side;
+// Whether cells (x0, y0) .. (x0 + 1, y0 + 1) lie in the grid: a negative
+// coordinate is a large unsigned one.
+__device__ inline bool in_grid(int x0, int y0, uint32_t w, uint32_t h) {
+  return static_cast<uint32_t>(x0) < w - 1u && static_cast<uint32_t>(y0) < h - 1u;
 }
-constexpr uint32_t kMinStagedAgents = 256;  // sparser tiles read global memory
+
+// The |T| values of the four cells around a sample's point (any values where the
+// point is outside the grid: !in), and the bilinear weights.
+struct Cells {
+  float v00, v10, v01, v11;
+  bool in;
+};
+struct Weights {
+  float dx, dy;
+};
+__device__ inline float mix_cells(const Cells& c, const Weights& f) {
+  const float v0 = wgsl_mix(c.v00, c.v10, f.dx);
+  const float v1 = wgsl_mix(c.v01, c.v11, f.dx);
+  return wgsl_mix(v0, v1, f.dy);
+}
+
+// Taps from a tile's window of the trail staged in LDS as f32 |T| (tile
+// windows, below), for points whose cells the caller knows to lie in the window
+// where they lie in the grid.  One 32-bit address serves a sample: the two cells
+// of a row are neighbours and the row below is `pitch` bytes on.
+template <int S>
+struct TileTaps {
+  using elem = typename TrailRead<S>::elem;
+  void* t;
+  uint32_t w, h;
+  const char* win;   // LDS
+  uint32_t pitch;    // bytes per window row
+  uint32_t origin;   // byte offset of the map's cell (0, 0) (mod 2^32)
+  __device__ Cells cells_inside(uint32_t x0, uint32_t y0) const {
+    const char* p = win + (__umul24(y0, pitch) + (x0 * 4u + origin));
+    const float* row = reinterpret_cast<const float*>(p);
+    const float* below = reinterpret_cast<const float*>(p + pitch);
+    return {fabsf(row[0]), fabsf(row[1]), fabsf(below[0]), fabsf(below[1]), true};
+  }
+  __device__ Cells cells(int x0, int y0) const {
+    const bool in = in_grid(x0, y0, w, h);
+    const uint32_t o = __umul24(static_cast<uint32_t>(y0), pitch) +
+                       (static_cast<uint32_t>(x0) * 4u + origin);
+    const char* p = win + (in ? o : 0u);
+    const float* row = reinterpret_cast<const float*>(p);
+    const float* below = reinterpret_cast<const float*>(p + pitch);
+    return {fabsf(row[0]), fabsf(row[1]), fabsf(below[0]), fabsf(below[1]), in};
+  }
+  __device__ Mark mark(uint32_t x, uint32_t y) const {
+    uint16_t* p = half_cell(x, y);
+    return {p, *p};
+  }
+  // The cell's |T| is in the window: the mark needs no load from the trail.
+  // (Marking in the window and storing the marked cells a row per wave at the
+  // workgroup's end measured 2% faster to 5% slower.)
+  __device__ Mark mark_inside(uint32_t x, uint32_t y) const {
+    const char* p = win + (__umul24(y, pitch) + (x * 4u + origin));
+    uint32_t raw;
+    if constexpr (S == SLM_STORAGE_F16)
+      raw = __builtin_bit_cast(uint16_t,
+                               static_cast<_Float16>(*reinterpret_cast<const float*>(p)));
+    else
+      raw = *reinterpret_cast<const uint16_t*>(p + 2);
+    return {half_cell(x, y), raw};
+  }
+  // The 16 bits that hold a cell's sign, in a trail below 2^32 bytes with rows
+  // below 2^24 (tile_staged).
+  __device__ uint16_t* half_cell(uint32_t x, uint32_t y) const {
+    constexpr uint32_t kBytes = sizeof(elem);
+    const uint32_t o = __umul24(y, w * kBytes) + (x * kBytes + (kBytes - 2u));
+    return reinterpret_cast<uint16_t*>(static_cast<char*>(t) + o);
+  }
+};
+
+// The cells around (px, py) and their weights.  kInside: the point is known to
+// lie in the grid with its neighbour cells; truncation is the floor of a value
+// >= 0, and v_fract is exact there.
+template <bool kInside, class Taps>
+__device__ inline Cells tap(const Taps& taps, float px, float py, Weights& f) {
+  if constexpr (kInside) {
+    f = {__builtin_amdgcn_fractf(px), __builtin_amdgcn_fractf(py)};
+    return taps.cells_inside(static_cast<uint32_t>(static_cast<int>(px)),
+                             static_cast<uint32_t>(static_cast<int>(py)));
+  } else {
+    const float fx = __builtin_floorf(px), fy = __builtin_floorf(py);
+    f = {px - fx, py - fy};
+    return taps.cells(static_cast<int>(fx), static_cast<int>(fy));
+  }
+}
+template <bool kInside, class Taps>
+__device__ inline Cells tap(const Taps& taps, double px, double py, Weights& f) {
+  if constexpr (kInside) {
+    f = {static_cast<float>(__builtin_amdgcn_fract(px)),
+         static_cast<float>(__builtin_amdgcn_fract(py))};
+    return taps.cells_inside(static_cast<uint32_t>(static_cast<int>(px)),
+                             static_cast<uint32_t>(static_cast<int>(py)));
+  } else {
+    const double fx = __builtin_floor(px), fy = __builtin_floor(py);
+    f = {static_cast<float>(px - fx), static_cast<float>(py - fy)};
+    return taps.cells(static_cast<int>(fx), static_cast<int>(fy));
+  }
+}
+
+// wgsl_mod with a second short case: when |a| < 2b, a/b truncates to +-1 (the
+// quotient is at most pred(2), as pred(2b)/b is) and a - b*(+-1) is a -+ b.  The
+// result is never -0.
+__device__ inline float mod_near(float a, float b) {
+  if (__builtin_fabsf(a) >= b && __builtin_fabsf(a) < b + b) return a - __builtin_copysignf(b, a);
+  return wgsl_mod(a, b);
+}
+// r + (r < 0 ? b : 0) for a result r of mod_near: r is never -0, so its sign
+// bit is the test, and adding +0 leaves the others.
+__device__ inline float wrap_up(float r, float b) {
+  uint32_t below;  // all ones below 0 (as asm: the compiler makes a compare and a select of it)
+  asm("v_ashrrev_i32 %0, 31, %1" : "=v"(below) : "v"(r));
+  return r + __uint_as_float(__float_as_uint(b) & below);
+}
+// `turn` for |angle| < kQuickAngle and turn_speed <= kQuickTurn: the distance to
+// either target is then 2 pi to within 2.5e-4, above turn_speed, so the turn is
+// -turn_speed or +turn_speed, the sign of rv - lv (exact: f32 subtraction keeps
+// denormals, so it is 0 only for equal values).
+__device__ inline float turn_quick(float angle, float lv, float rv, float cv, float turn_speed,
+                                   uint32_t sign) {
+  const float d = rv - lv;
+  const float turned =
+      angle + __uint_as_float(__float_as_uint(turn_speed) ^ (__float_as_uint(d) & sign));
+  const bool straight = (d == 0.0f) | ((cv > lv) & (cv > rv));
+  return straight ? angle : turned;
+}
+
+// jitter_term with the middle range's shorter reduction.
+__device__ inline float jitter_term_mid(uint32_t index, float x, float y, float jitter) {
+  float hx = static_cast<float>(static_cast<int32_t>(index)) * 12.9898f;
+  hx = hx + x * 78.233f;
+  hx = hx + y * 37.719f;
+  const float ax = __builtin_fabsf(hx);
+  float s, c;
+  // waves wholly inside the middle range, all but a few, take its shorter form
+  if (__all(ax >= SLM_TRIG_SMALL_MAX && ax < SLM_TRIG_MID_MAX))
+    s = slm_sinf_mid(hx);
+  else
+    slm_sincosf_finite(hx, &s, &c);  // finite: index, positions and products are bounded
+  float v = s * 43758.5453f;
+  float rnd = v - __builtin_floorf(v);
+  return (rnd * 2.0f - 1.0f) * jitter;
+}
+
+// The agent arrays from slot `base` on (uniform), indexed by a lane's small
+// offset: scalar bases and 32-bit lane offsets.
+__device__ inline AgentSoA agents_from(const AgentSoA& a, uint32_t base, bool p64) {
+  AgentSoA r = a;
+  if (p64) {
+    r.x64 += base;
+    r.y64 += base;
+  } else {
+    r.x += base;
+    r.y += base;
+  }
+  r.th += base;
+  r.v += base;
+  if (r.id) r.id += base;
+  return r;
+}
+
+// Element j of an array at a uniform address: scalar base, 32-bit byte offset.
+template <class T>
+__device__ inline T& lane_at(T* base, uint32_t j) {
+  return *reinterpret_cast<T*>(reinterpret_cast<char*>(base) + j * static_cast<uint32_t>(sizeof(T)));
+}
+
+template <bool P64>
+__device__ inline AgentState<P64> load_lane(const AgentSoA& a, uint32_t j) {
+  AgentState<P64> st;
+  st.angle = lane_at(a.th, j);
+  st.speed = lane_at(a.v, j);
+  if (P64) {
+    st.xd = lane_at(a.x64, j);
+    st.yd = lane_at(a.y64, j);
+    st.x = st.y = 0.0f;
+  } else {
+    st.xd = st.yd = 0.0;
+    st.x = lane_at(a.x, j);
+    st.y = lane_at(a.y, j);
+  }
+  return st;
+}
+
+constexpr float kQuickAngle = 2048.0f;
+constexpr float kQuickSensorAngle = 1024.0f;  // angle +- it stays below SLM_TRIG_SMALL_MAX
+constexpr float kQuickTurn = 6.25f;           // below 2 pi - 2.5e-4
+
+__device__ inline float in_vgpr(float v) {
+  asm("" : "+v"(v));
+  return v;
+}
+
+// Uniform values of one instance's updates.
+struct UpdateConsts {
+  bool ordinary;          // parameters in the ordinary range
+  float sa, sd, turn;
+  float two_over_pi, pio2_c1;  // slm_sincosf_small_k's constants
+  uint32_t sign;
+  __device__ void sincos(float v, float* s, float* c) const {
+    slm_sincosf_small_k(v, two_over_pi, pio2_c1, sign, s, c);
+  }
+};
+
+__device__ inline UpdateConsts update_consts(const DevParams& p) {
+  UpdateConsts k;
+  k.ordinary = __builtin_fabsf(p.sensor_angle) <= kQuickSensorAngle && p.turn <= kQuickTurn &&
+               p.speed_min <= p.speed_max;
+  k.sa = in_vgpr(p.sensor_angle);
+  k.sd = in_vgpr(p.sensor_dist);
+  k.turn = in_vgpr(p.turn);
+  k.two_over_pi = in_vgpr(SLM_TWO_OVER_PI_F);
+  k.pio2_c1 = in_vgpr(SLM_PIO2_C1);
+  k.sign = __float_as_uint(in_vgpr(-0.0f));
+  return k;
+}
+
+// Has the loads of `st` counted as done here: they were issued before loads
+// that have been waited for, and behind the stores that follow, a wait for
+// them would be a wait for the stores.
+template <bool P64>
+__device__ inline void wait_state(AgentState<P64>& st) {
+  asm volatile("" : "+v"(st.angle), "+v"(st.speed));
+  if constexpr (P64)
+    asm volatile("" : "+v"(st.xd), "+v"(st.yd));
+  else
+    asm volatile("" : "+v"(st.x), "+v"(st.y));
+}
+
+// One agent (lane offset j of `a`, state st, instance slot `slot`) for one
+// step; nxt: the state in flight for the lane's next agent.
+template <bool P64, bool kInside, class Taps>
+__device__ inline void tile_update(const AgentSoA& a, uint32_t j, uint32_t slot,
+                                   const AgentState<P64>& st, AgentState<P64>& nxt,
+                                   const Instance& in, const DevParams& p, const Taps& taps,
+                                   const UpdateConsts& k) {
+  const uint32_t w = in.width, h = in.height;
+  float angle = st.angle, speed = st.speed;
+  double xd = st.xd, yd = st.yd;
+  float x = P64 ? static_cast<float>(xd) : st.x, y = P64 ? static_cast<float>(yd) : st.y;
+
+  // :72; the median is the clamp where speed_min <= speed_max
+  float sp = __builtin_amdgcn_fmed3f(speed, p.speed_min, p.speed_max);
+  if (sp != speed) lane_at(a.v, j) = sp;
+  speed = sp;
+
+  float al = angle - k.sa, ar = angle + k.sa;  // :75-77
+  float sl, cl, sr, cr, sc, cc;
+  k.sincos(al, &sl, &cl);
+  k.sincos(ar, &sr, &cr);
+  k.sincos(angle, &sc, &cc);
+  const float sd = k.sd;
+  Cells lc, rc, cc4;
+  Weights lf, rf, cf;
+  __builtin_amdgcn_s_setprio(2);
+  if constexpr (P64) {
+    lc = tap<kInside>(taps, xd + static_cast<double>(sd * cl), yd + static_cast<double>(sd * sl), lf);
+    rc = tap<kInside>(taps, xd + static_cast<double>(sd * cr), yd + static_cast<double>(sd * sr), rf);
+    cc4 = tap<kInside>(taps, xd + static_cast<double>(sd * cc), yd + static_cast<double>(sd * sc), cf);
+  } else {
+    lc = tap<kInside>(taps, x + sd * cl, y + sd * sl, lf);  // :79-95, read order L, R, C
+    rc = tap<kInside>(taps, x + sd * cr, y + sd * sr, rf);
+    cc4 = tap<kInside>(taps, x + sd * cc, y + sd * sc, cf);
+  }
+  const float lv = lc.in ? mix_cells(lc, lf) : 0.0f;
+  const float rv = rc.in ? mix_cells(rc, rf) : 0.0f;
+  const float cv = cc4.in ? mix_cells(cc4, cf) : 0.0f;
+  __builtin_amdgcn_s_setprio(0);
+  angle = turn_quick(angle, lv, rv, cv, k.turn, k.sign);
+
+  // With zero jitter the term is (finite) * 0 = +-0, which leaves the angle
+  // unchanged, so the hash (and the original-index load) is skipped.
+  if (p.jitter != 0.0f) {
+    uint32_t index = a.id ? lane_at(a.id, j) : slot;  // S6
+    angle += jitter_term_mid(index, x, y, p.jitter);
+  }
+
+  angle = wrap_up(mod_near(angle, kTau), kTau);  // :121-122; now in [0, 2 pi]
+
+  float move = speed * kTimeStep;  // :125-127
+  float ms, mc;
+  k.sincos(angle, &ms, &mc);
+  int dx, dy;
+  if (P64) {
+    xd = xd + static_cast<double>(move * mc);
+    yd = yd + static_cast<double>(move * ms);
+    if (!kInside) {
+      double fw = static_cast<double>(w), fh = static_cast<double>(h);
+      xd = mod64(xd, fw);
+      if (xd < 0.0) xd = xd + fw;
+      yd = mod64(yd, fh);
+      if (yd < 0.0) yd = yd + fh;
+    }
+    dx = static_cast<int>(xd);
+    dy = static_cast<int>(yd);
+  } else {
+    x = x + move * mc;
+    y = y + move * ms;
+    if (!kInside) {
+      float fw = static_cast<float>(w), fh = static_cast<float>(h);  // :130-133
+      x = wrap_up(mod_near(x, fw), fw);
+      y = wrap_up(mod_near(y, fh), fh);
+    }
+    dx = static_cast<int>(x);
+    dy = static_cast<int>(y);
+  }
+  // The mark (:136-141): its load (clipped windows only), the state's stores, its store.
+  __builtin_amdgcn_s_setprio(2);
+  const uint32_t ux = static_cast<uint32_t>(dx), uy = static_cast<uint32_t>(dy);
+  bool in_map = true;
+  Mark mark{};
+  if constexpr (kInside) {
+    mark = taps.mark_inside(ux, uy);
+  } else {
+    in_map = ux < w && uy < h;  // wrapped positions are >= 0
+    if (in_map) mark = taps.mark(ux, uy);
+  }
+  wait_state(nxt);
+  if constexpr (P64) {
+    lane_at(a.x64, j) = xd;  // :144
+    lane_at(a.y64, j) = yd;
+  } else {
+    lane_at(a.x, j) = x;
+    lane_at(a.y, j) = y;
+  }
+  lane_at(a.th, j) = angle;
+  if (in_map) mark.store();
+  __builtin_amdgcn_s_setprio(0);
+}
+
+template <bool P64>
+constexpr int kTileBlockOf = P64 ? 512 : 1024;
+constexpr uint32_t kMinStagedAgents = 256;  // sparser items read global memory
 
 __device__ inline uint32_t compact_bits(uint32_t v) {  // even bits -> 16 bits
   v &= 0x55555555u;
@@ -700,75 +1028,138 @@ __device__ inline uint32_t compact_bits(uint32_t v) {  // even bits -> 16 bits
 struct TiledArgs {
   AgentSoA a;
   void* trail;
-  const Instance* inst;
-  const DevParams* params;
   const WorkItem* items;
-  const uint32_t* item_total;
-  uint32_t side;        // LDS window side limit (cells)
-  uint32_t resort;      // steps between re-sorts
-  int xcd_remap;
+  uint32_t drift_steps;  // steps since the re-sort, this one included
 };
 
-template <int S, bool P64>
-__global__ __launch_bounds__(kTiledBlock) void agents_tiled_kernel(TiledArgs args) {
-  using elem = typename TrailRead<S>::elem;
-  extern __shared__ __align__(16) unsigned char smem[];
-  elem* win = reinterpret_cast<elem*>(smem);
-  uint32_t item = args.xcd_remap ? xcd_logical_block(blockIdx.x, gridDim.x) : blockIdx.x;
-  if (item >= *args.item_total) return;  // uniform per block
-  const WorkItem wi = args.items[item];
-  const Instance in = args.inst[wi.inst];
-  const DevParams p = args.params[wi.inst];
-  elem* trail = static_cast<elem*>(args.trail) + in.trail_off;
+// A work item's window: `rows` rows from y0 of `cpr` 16-byte chunks from x0,
+// chunk q of the window being chunk q % cpr of row q / cpr, and in LDS 16-byte
+// (f32) or 32-byte (16-bit formats, widened) entry q.
+struct TileWindow {
+  float cx, cy, half;       // agents with |x - cx| < half and |y - cy| < half sense inside it
+  int x0, y0, cpr, rows;
+  uint32_t inv_cpr;         // ceil(2^20 / cpr)
+  bool staged, clipped;
+};
+
+template <int S>
+__device__ inline TileWindow tile_window(const WorkItem& wi, const Instance& in,
+                                         const DevParams& p, uint32_t drift_steps) {
+  constexpr int V = static_cast<int>(16 / sizeof(typename TrailRead<S>::elem));
   const int tile = 1 << in.tile_log2;
   const int tx = static_cast<int>(compact_bits(wi.tile)) * tile;
   const int ty = static_cast<int>(compact_bits(wi.tile >> 1)) * tile;
-  // margin the window must cover: sensor reach + bilinear neighbour + drift
-  float reach = __builtin_ceilf(__builtin_fabsf(p.sensor_dist)) + 2.0f +
-                __builtin_ceilf(p.speed_max * kTimeStep * static_cast<float>(args.resort));
-  int room = (static_cast<int>(args.side) - tile) / 2;
-  bool staged = room > 0 && reach <= static_cast<float>(room) &&
-                wi.end - wi.begin >= kMinStagedAgents;  // uniform
-  if (!staged) {
-    GlobalTaps<S> taps{trail, in.width, in.height};
-    agent_loop<P64, kTiledBlock>(args.a, wi.begin, wi.end, in, p, taps);
-    return;
-  }
-  const int m = room;
-  const int wx0 = max(tx - m, 0), wx1 = min(tx + tile + m, static_cast<int>(in.width));
-  const int wy0 = max(ty - m, 0), wy1 = min(ty + tile + m, static_cast<int>(in.height));
-  const int ww = wx1 - wx0, wh = wy1 - wy0;
-  // Stage the window: wave w takes rows w, w + 16, ..., lane l columns l,
-  // l + 64, ...; every thread issues all of its loads before its LDS stores,
-  // so they are in flight together.
-  constexpr int kSide = window_side_of(sizeof(elem));
-  constexpr int kWaves = kTiledBlock / 64;
-  constexpr int kRows = (kSide + kWaves - 1) / kWaves;
-  constexpr int kCols = (kSide + 63) / 64;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  uint32_t v[kRows][kCols];
+  const TileReach r = tile_reach(p, drift_steps);
+  // uniform, but computed in vector registers: back to a scalar one
+  const int m = __builtin_amdgcn_readfirstlane(r.margin);
+  const TileExtent e = tile_extent(in, tx, ty, m, V);
+  TileWindow win;
+  win.x0 = e.x0;
+  win.y0 = e.y0;
+  win.cpr = e.cpr;
+  win.rows = e.rows;
+  // q * inv_cpr stays below 2^32 (rows <= 1024), and it >> 20 is q / cpr while
+  // q * cpr < 2^20
+  win.inv_cpr = ((1u << 20) + static_cast<uint32_t>(e.cpr) - 1u) / static_cast<uint32_t>(e.cpr);
+  win.clipped = tx - m < 0 || ty - m < 0 || tx + tile + m > static_cast<int>(in.width) ||
+                ty + tile + m > static_cast<int>(in.height);
+  win.staged = wi.end - wi.begin >= kMinStagedAgents && tile_staged(in, e, V);
+  win.cx = static_cast<float>(tx) + 0.5f * static_cast<float>(tile);
+  win.cy = static_cast<float>(ty) + 0.5f * static_cast<float>(tile);
+  win.half = win.staged ? 0.5f * static_cast<float>(tile) + static_cast<float>(m) - r.reach : -1.0f;
+  return win;
+}
+
+template <int S, bool P64, bool kOne>
+__global__ __launch_bounds__(kTileBlockOf<P64>)
+    __attribute__((amdgpu_waves_per_eu(P64 ? 4 : 8))) void agents_tiled_kernel(
+        TiledArgs args, const Instance* __restrict__ insts, const DevParams* __restrict__ params) {
+  using elem = typename TrailRead<S>::elem;
+  constexpr int V = static_cast<int>(16 / sizeof(elem));  // cells per 16-byte chunk
+  constexpr int kTileBlock = kTileBlockOf<P64>;
+  constexpr int kDeep = (static_cast<int>(kTileLds) / (V * 4) + kTileBlock - 1) / kTileBlock;  // chunks per lane
+  extern __shared__ __align__(16) char smem[];
+  const uint32_t t = threadIdx.x;
+  // kOne (a pool of one instance): the tables' loads do not wait for the item's
+  WorkItem wi = args.items[blockIdx.x];
+  Instance in = insts[kOne ? 0u : wi.inst];
+  DevParams p = params[kOne ? 0u : wi.inst];
+  if (wi.begin == wi.end) return;  // uniform: past the last item
+  elem* trail = static_cast<elem*>(args.trail) + in.trail_off;
+
+  AgentSoA here = agents_from(args.a, wi.begin, P64);
+  AgentState<P64> cur{};
+  if (t < wi.end - wi.begin) cur = load_lane<P64>(here, t);
+  const TileWindow win =
+      tile_window<S>(wi, in, p, args.drift_steps);
+  if (win.staged) {
+    const uint32_t n = static_cast<uint32_t>(win.cpr * win.rows);
+    const char* src = reinterpret_cast<const char*>(
+        trail + (static_cast<size_t>(win.y0) * in.width + static_cast<uint32_t>(win.x0)));
+    uint4 raw[kDeep];  // every chunk in flight before the first is stored
 #pragma unroll
-  for (int rr = 0; rr < kRows; rr++) {
-    int r = wave + rr * kWaves;
-    const elem* row = trail + static_cast<size_t>(wy0 + r) * in.width + wx0;
-#pragma unroll
-    for (int cc = 0; cc < kCols; cc++) {
-      int c = lane + cc * 64;
-      v[rr][cc] = (r < wh && c < ww) ? static_cast<uint32_t>(row[c]) : 0u;
+    for (int k = 0; k < kDeep; k++) {
+      const uint32_t q = min(t + k * kTileBlock, n - 1u);
+      const uint32_t r = (q * win.inv_cpr) >> 20;
+      const uint32_t c = q - __umul24(r, static_cast<uint32_t>(win.cpr));
+      uint4 v;
+      __builtin_memcpy(&v, src + (__umul24(r, in.width) + c * V) * static_cast<uint32_t>(sizeof(elem)),
+                       sizeof v);
+      raw[k] = v;
     }
-  }
 #pragma unroll
-  for (int rr = 0; rr < kRows; rr++) {
-    int r = wave + rr * kWaves;
+    for (int k = 0; k < kDeep; k++) {
+      const uint32_t q = t + k * kTileBlock;
+      if (q < n) {
+        const uint32_t u[4] = {raw[k].x, raw[k].y, raw[k].z, raw[k].w};
+        if constexpr (V == 4) {  // marks included: the taps read |T|
+          reinterpret_cast<uint4*>(smem)[q] = make_uint4(u[0], u[1], u[2], u[3]);
+        } else {
+          float f[8];
 #pragma unroll
-    for (int cc = 0; cc < kCols; cc++) {
-      int c = lane + cc * 64;
-      if (r < wh && c < ww) win[r * ww + c] = static_cast<elem>(v[rr][cc] & ~TrailRead<S>::kSign);
+          for (int i = 0; i < 4; i++) TrailRead<S>::split(u[i], f[2 * i], f[2 * i + 1]);
+          reinterpret_cast<float4*>(smem)[2 * q] = make_float4(f[0], f[1], f[2], f[3]);
+          reinterpret_cast<float4*>(smem)[2 * q + 1] = make_float4(f[4], f[5], f[6], f[7]);
+        }
+      }
     }
   }
   __syncthreads();
-  WindowTaps<S> taps{trail, in.width, in.height, win, wx0, wy0, ww, wh};
-  agent_loop<P64, kTiledBlock>(args.a, wi.begin, wi.end, in, p, taps);
+  const uint32_t pitch = static_cast<uint32_t>(win.cpr) * (V * 4u);
+  const TileTaps<S> taps{trail, in.width, in.height, smem, pitch,
+                         0u - (static_cast<uint32_t>(win.y0) * pitch +
+                               static_cast<uint32_t>(win.x0) * 4u)};
+  const GlobalTaps<S> global{trail, in.width, in.height};
+  const UpdateConsts k = update_consts(p);
+  const float cx = in_vgpr(win.cx), cy = in_vgpr(win.cy);
+  const uint32_t count = wi.end - wi.begin;
+  const uint32_t first_slot = wi.begin - in.agent_off;
+  for (uint32_t j = t;;) {
+    const uint32_t nj = j + kTileBlock;
+    AgentState<P64> nxt = cur;
+    if (nj < count) nxt = load_lane<P64>(here, nj);
+    if (j >= count) break;
+    const float x = P64 ? static_cast<float>(cur.xd) : cur.x;
+    const float y = P64 ? static_cast<float>(cur.yd) : cur.y;
+    const bool ordinary = k.ordinary && __builtin_fabsf(cur.angle) < kQuickAngle;
+    const uint32_t slot = first_slot + j;
+    if (__all(ordinary && __builtin_fabsf(x - cx) < win.half &&
+              __builtin_fabsf(y - cy) < win.half)) {
+      if (!win.clipped)
+        tile_update<P64, true>(here, j, slot, cur, nxt, in, p, taps, k);
+      else
+        tile_update<P64, false>(here, j, slot, cur, nxt, in, p, taps, k);
+    } else {
+      AgentState<P64> st = cur;
+      if (P64) {
+        st.x = x;
+        st.y = y;
+      }
+      agent_update<P64>(args.a, wi.begin + j, st, in, p, global);
+    }
+    j = nj;
+    cur = nxt;
+  }
 }
 
 // ---- initialisation ------------------------------------------------------
@@ -925,8 +1316,6 @@ void launch_agents(const Pool& pool, const AgentSoA& a, void* trail, hipStream_t
   }
 }
 
-uint32_t window_side(int storage) { return window_side_of(storage_bytes(storage)); }
-
 void prime_persistent_agents() {
   auto each = [](auto s_tag) {
     constexpr int S = decltype(s_tag)::value;
@@ -940,29 +1329,35 @@ void prime_persistent_agents() {
   each(std::integral_constant<int, SLM_STORAGE_F16>{});
 }
 
-void launch_agents_tiled(const Pool& pool, const AgentSoA& a, void* trail, hipStream_t stream) {
+void launch_agents_tiled(const Pool& pool, const AgentSoA& a, void* trail, uint32_t drift_steps,
+                         hipStream_t stream) {
   if (pool.total_agents == 0 || pool.max_items == 0) return;
-  TiledArgs args{a,          trail,           pool.inst,    pool.params, pool.items,
-                 pool.item_total, window_side(pool.storage), pool.resort_interval, pool.xcd_remap};
-  size_t lds = kWindowBytes;
-  uint32_t nb = pool.max_items;
-#define SLM_TILED(S)                                                                 \
-  if (pool.pos64)                                                                    \
-    agents_tiled_kernel<S, true><<<nb, kTiledBlock, lds, stream>>>(args);            \
-  else                                                                               \
-    agents_tiled_kernel<S, false><<<nb, kTiledBlock, lds, stream>>>(args)
+  const int block = pool.pos64 ? kTileBlockOf<true> : kTileBlockOf<false>;
+  TiledArgs args{a, trail, pool.items, drift_steps};
+  auto go = [&](auto* one, auto* many) {
+    if (pool.count == 1)
+      one<<<pool.max_items, block, kTileLds, stream>>>(args, pool.inst, pool.params);
+    else
+      many<<<pool.max_items, block, kTileLds, stream>>>(args, pool.inst, pool.params);
+  };
+  auto storage = [&](auto s_tag) {
+    constexpr int S = decltype(s_tag)::value;
+    if (pool.pos64)
+      go(agents_tiled_kernel<S, true, true>, agents_tiled_kernel<S, true, false>);
+    else
+      go(agents_tiled_kernel<S, false, true>, agents_tiled_kernel<S, false, false>);
+  };
   switch (pool.storage) {
     case SLM_STORAGE_BF16:
-      SLM_TILED(SLM_STORAGE_BF16);
+      storage(std::integral_constant<int, SLM_STORAGE_BF16>{});
       break;
     case SLM_STORAGE_F16:
-      SLM_TILED(SLM_STORAGE_F16);
+      storage(std::integral_constant<int, SLM_STORAGE_F16>{});
       break;
     default:
-      SLM_TILED(SLM_STORAGE_F32);
+      storage(std::integral_constant<int, SLM_STORAGE_F32>{});
       break;
   }
-#undef SLM_TILED
 }
 
 void launch_init_agents(const Instance& in, const AgentSoA& a, int pos64, uint64_t seed,

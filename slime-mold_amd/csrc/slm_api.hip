@@ -14,6 +14,7 @@
 // starts, so at most four exist per handle.  Every entry point validates its
 // arguments before any kernel is launched, so the kernels can rely on
 // in-range shapes and finite, bounded positions.
+#include <algorithm>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -340,10 +341,8 @@ class Engine {
     p.tile_inst = tile_inst_d_;
     // the re-sort builds the tiled pass's work list only when that pass is on
     // (turning it on re-lays the tables and waits for the next re-sort)
-    p.items = (cfg.flags & SLM_FLAG_TILED_SENSING) ? items_d_ : nullptr;
-    p.item_total = item_total_d_;
+    p.items = (cfg.flags & SLM_FLAG_TILED_SENSING) || auto_tiles() ? items_d_ : nullptr;
     p.max_items = max_items_;
-    p.resort_interval = cfg.resort_interval;
     p.agents_per_group = cfg.agents_per_group;
     p.preload_rows = preload_rows_;
     p.stochastic_rounding = (cfg.flags & SLM_FLAG_STOCHASTIC_ROUNDING) ? 1 : 0;
@@ -366,8 +365,7 @@ class Engine {
         SLM_TRY(run_chunk_graph());
         n -= chunk;
       } else {  // fewer than a chunk left, or no graphs: launch them directly
-        const uint64_t s0 = steps_done;
-        enqueue_steps(n, [&](uint32_t j) { return sort_due(s0 + j); });
+        enqueue_steps(steps_done, n);
         steps_done += n;
         n = 0;
       }
@@ -425,6 +423,18 @@ class Engine {
         const bool replan = gauss_th(cfg.storage, c) != gauss_th(cfg.storage, gauss_rclass_);
         gauss_rclass_ = c;
         if (replan) return relayout(layout_trail_tables());
+      }
+    }
+    // captured chunks hold the sensing of the parameters they were captured under
+    // (their results hold for any): recapture where another one pays
+    const uint32_t fits = auto_tiles() ? window_steps(k) : 0u;
+    if (fits != window_steps_[k]) {
+      window_steps_[k] = fits;
+      const uint32_t tiles = tile_steps_now();
+      if (tiles != tile_steps_) {
+        SLM_HIP(hipStreamSynchronize(stream));
+        drop_graphs();
+        tile_steps_ = tiles;
       }
     }
     return SLM_OK;
@@ -807,7 +817,7 @@ class Engine {
       launch_render(a, lut, cfg.storage, stream);
     };
     if (steps) {
-      enqueue_step(sort_due(steps_done), draw);
+      enqueue_step(steps_done, draw);
       steps_done++;
     } else {
       draw();
@@ -952,7 +962,7 @@ class Engine {
     // the timed window starts with a re-sort of agents that drifted a whole
     // interval, as in a long run.
     steps_done = 0;
-    enqueue_steps(kTuneSpan, [&](uint32_t j) { return sort_due(j); });
+    enqueue_steps(0, kTuneSpan);
     steps_done = kTuneSpan;
     uint32_t n = (steps + kTuneSpan - 1) / kTuneSpan * kTuneSpan;
     // The step time is the device span of n steps captured as one graph, as
@@ -962,7 +972,7 @@ class Engine {
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     SLM_HIP(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
-    enqueue_steps(n, [&](uint32_t j) { return sort_due(kTuneSpan + j); });
+    enqueue_steps(kTuneSpan, n);
     hipError_t ce = hipStreamEndCapture(stream, &graph);
     if (ce == hipSuccess) ce = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
     if (graph) (void)hipGraphDestroy(graph);
@@ -1134,9 +1144,11 @@ class Engine {
   uint32_t total_gtiles_ = 0;  // Gaussian-pass tiles
   int gauss_rclass_ = kGaussMaxR;  // Gaussian-pass LDS radius class (gauss_class)
   uint32_t preload_rows_ = 0;
+  uint64_t total_cells_ = 0;
+  std::vector<uint32_t> window_steps_;  // per instance, for the current layout and parameters
+  uint32_t tile_steps_ = 0;             // tile_steps_now for them
   uint32_t* tile_inst_d_ = nullptr;
   WorkItem* items_d_ = nullptr;
-  uint32_t* item_total_d_ = nullptr;
   bool tiles_ready_ = false;  // the latest re-sort's work list matches the layout
   uint64_t trail_elems_ = 0;
   // Captured chunks.  A chunk's launches depend on the current trail and
@@ -1385,8 +1397,13 @@ class Engine {
       first = false;
     }
     total_bins_ = sorting() ? static_cast<uint32_t>(bins) : 0;
+    total_cells_ = total_cells;
     SLM_HIP(hipMemcpy(inst_d_, inst.data(), inst.size() * sizeof(Instance), hipMemcpyHostToDevice));
     SLM_TRY(build_groups());
+    window_steps_.assign(spec.size(), 0u);
+    if (auto_tiles())
+      for (size_t k = 0; k < spec.size(); k++) window_steps_[k] = window_steps(k);
+    tile_steps_ = tile_steps_now();
 
     dev_free(unit_block_d_);
     uint32_t nb = blocks_for(units, kTrailWavesPerBlock);
@@ -1407,9 +1424,8 @@ class Engine {
     dev_free(scan_levels_);
     dev_free(tile_inst_d_);
     dev_free(items_d_);
-    dev_free(item_total_d_);
     sort_.count = sort_.offset = sort_.tile_items = scan_levels_ = nullptr;
-    tile_inst_d_ = item_total_d_ = nullptr;
+    tile_inst_d_ = nullptr;
     items_d_ = nullptr;
     total_tiles_ = max_items_ = 0;
     if (sorting()) {
@@ -1426,8 +1442,6 @@ class Engine {
       SLM_HIP(hipMemcpy(tile_inst_d_, tmap.data(), tmap.size() * 4ull, hipMemcpyHostToDevice));
       SLM_TRY(dev_alloc(&sort_.tile_items, total_tiles_ * 4ull));
       SLM_TRY(dev_alloc(&items_d_, max_items_ * sizeof(WorkItem)));
-      SLM_TRY(dev_alloc(&item_total_d_, 4));
-      SLM_HIP(hipMemset(item_total_d_, 0, 4));
       uint32_t lv = plan_scan(sort_, total_bins_);
       SLM_TRY(dev_alloc(&scan_levels_, lv * 4ull));
       uint32_t at = 0;
@@ -1454,32 +1468,90 @@ class Engine {
     return sorting() && step_index % cfg.resort_interval == 0;
   }
 
-  // Tiled sensing (when asked for) once a re-sort has laid agents out by
-  // tile; otherwise the global-memory pass.  Both give the same bits.
-  void enqueue_agents(const Pool& p) {
-    if (sorting() && tiles_ready_ && (cfg.flags & SLM_FLAG_TILED_SENSING))
-      launch_agents_tiled(p, agents_[acur_], trail_[cur_], stream);
+  // Whether the pool's agents sense through tile windows of the library's own
+  // accord: with the plain re-sort key, one launch per pass over the pool and no
+  // other sensing asked for, from 2^21 agents on and one agent to four cells.
+  // Measured (us per agent pass, global against tiled, re-sort every 20 steps):
+  // 2048^2 with 2^21 agents 38.8 against 31.6, with 2^20 25.0 either way, with
+  // 2^19 19.8 against 21.3; 4096^2 with 2^24 293 against 221, with 2^23 128
+  // against 109, with 2^22 (a quarter per cell) 77.7 against 78.2 and 69.4
+  // against 66.0; 256^2 with 2^18 17.4 against 20.4: fewer agents do not fill
+  // the chip with 1024-thread workgroups, sparser ones stage cells that few read.
+  bool auto_tiles() const {
+    constexpr uint32_t kMinAgents = 1u << 21;
+    return sorting() && groups_.size() <= 1 && cfg.sort_key == 0u &&
+           !(cfg.flags & (SLM_FLAG_WINDOW_SENSING | SLM_FLAG_PERSISTENT)) &&
+           total_agents_ >= kMinAgents && total_agents_ >= total_cells_ / 4u;
+  }
+
+  // The most steps after a re-sort, up to the interval, at which instance k's tile
+  // windows can be staged (0: never, as with sensors that reach hundreds of cells).
+  uint32_t window_steps(size_t k) const {
+    const Instance& in = inst[k];
+    const DevParams dp = make_dev_params(spec[k].params);
+    const int V = cfg.storage == SLM_STORAGE_F32 ? 4 : 8;
+    const int tile = 1 << in.tile_log2;
+    // a tile in the middle has the largest window
+    const int tx = static_cast<int>(in.width) / 2 / tile * tile;
+    const int ty = static_cast<int>(in.height) / 2 / tile * tile;
+    uint32_t lo = 0, hi = std::min<uint32_t>(cfg.resort_interval, 4096u);
+    while (lo < hi) {  // windows grow with the steps
+      const uint32_t mid = (lo + hi + 1u) / 2u;
+      if (tile_staged(in, tile_extent(in, tx, ty, tile_reach(dp, mid).margin, V), V))
+        lo = mid;
+      else
+        hi = mid - 1u;
+    }
+    return lo;
+  }
+
+  // The most steps after a re-sort at which at least half of the agents sense
+  // through windows; 0 where the pool does not.
+  uint32_t tile_steps_now() const {
+    if (!auto_tiles()) return 0;
+    std::vector<std::pair<uint32_t, uint64_t>> by_steps;
+    for (size_t k = 0; k < spec.size(); k++) by_steps.push_back({window_steps_[k], spec[k].agents});
+    std::sort(by_steps.begin(), by_steps.end());
+    uint64_t agents = 0;
+    while (!by_steps.empty()) {
+      agents += by_steps.back().second;
+      if (agents * 2u >= total_agents_) return by_steps.back().first;
+      by_steps.pop_back();
+    }
+    return 0;
+  }
+
+  // Tiled sensing (when asked for, or where it pays: auto_tiles) once a re-sort
+  // has laid agents out by tile; otherwise the global-memory pass.  Both give
+  // the same bits.
+  void enqueue_agents(const Pool& p, uint64_t step) {
+    const uint32_t drift = sorting() ? static_cast<uint32_t>(step % cfg.resort_interval) + 1u : 0u;
+    if (sorting() && tiles_ready_ &&
+        ((cfg.flags & SLM_FLAG_TILED_SENSING) || drift <= tile_steps_))
+      launch_agents_tiled(p, agents_[acur_], trail_[cur_], drift, stream);
     else
       launch_agents(p, agents_[acur_], trail_[cur_], stream);
   }
 
-  // One step; `between` runs after the agent pass is enqueued and before the
-  // trail pass (the reference's display point).
+  void enqueue_sort(const Pool& p) {
+    launch_morton_sort(p, agents_[acur_], agents_[acur_ ^ 1], sort_, stream);
+    acur_ ^= 1;
+    tiles_ready_ = true;
+  }
+
+  // Absolute step `step`; `between` runs after the agent pass is enqueued and
+  // before the trail pass (the reference's display point).
   template <class Between>
-  void enqueue_step(bool do_sort, Between&& between) {
+  void enqueue_step(uint64_t step, Between&& between) {
     Pool p = pool();
-    if (do_sort && sorting() && total_agents_ > 0) {
-      launch_morton_sort(p, agents_[acur_], agents_[acur_ ^ 1], sort_, stream);
-      acur_ ^= 1;
-      tiles_ready_ = true;
-    }
-    enqueue_agents(p);
+    if (sorts_at(step)) enqueue_sort(p);
+    enqueue_agents(p, step);
     between();
     launch_trail(p, trail_[cur_], trail_[cur_ ^ 1], stream);
     cur_ ^= 1;
   }
-  void enqueue_step(bool do_sort) {
-    enqueue_step(do_sort, [] {});
+  void enqueue_step(uint64_t step) {
+    enqueue_step(step, [] {});
   }
 
   // ---- instance groups ---------------------------------------------------------
@@ -1659,24 +1731,19 @@ class Engine {
     return static_cast<char*>(trail_[buf]) + elem * storage_bytes(cfg.storage);
   }
 
-  // Enqueues n steps; sorts(j) says whether step j re-sorts first.  With
-  // instance groups, each stretch between re-sorts forks onto the group
-  // streams and joins back before the next re-sort (or the end).
-  template <class SortAt>
-  void enqueue_steps(uint32_t n, SortAt&& sorts) {
+  // Enqueues n steps from absolute step s0 on.  With instance groups, each
+  // stretch between re-sorts forks onto the group streams and joins back before
+  // the next re-sort (or the end).
+  void enqueue_steps(uint64_t s0, uint32_t n) {
     if (groups_.size() <= 1) {
-      for (uint32_t j = 0; j < n; j++) enqueue_step(sorts(j));
+      for (uint32_t j = 0; j < n; j++) enqueue_step(s0 + j);
       return;
     }
     uint32_t j = 0;
     while (j < n) {
-      if (sorts(j) && sorting() && total_agents_ > 0) {
-        launch_morton_sort(pool(), agents_[acur_], agents_[acur_ ^ 1], sort_, stream);
-        acur_ ^= 1;
-        tiles_ready_ = true;
-      }
+      if (sorts_at(s0 + j)) enqueue_sort(pool());
       uint32_t m = 1;
-      while (j + m < n && !sorts(j + m)) m++;
+      while (j + m < n && !sorts_at(s0 + j + m)) m++;
       // group g runs on stream g % L (0: the engine's stream)
       const size_t L = std::min<size_t>(groups_.size(), kGroupStreams);
       (void)hipEventRecord(fork_ev_, stream);
@@ -1732,7 +1799,7 @@ class Engine {
       int cur0 = cur_, acur0 = acur_;
       hipGraph_t graph = nullptr;
       SLM_HIP(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
-      enqueue_steps(chunk, [&](uint32_t j) { return sorts_at(s0 + j); });
+      enqueue_steps(s0, chunk);
       hipError_t e = hipStreamEndCapture(stream, &graph);
       cur_ = cur0;
       acur_ = acur0;
@@ -1752,19 +1819,17 @@ class Engine {
     return SLM_OK;
   }
 
-  // Enqueues one step with events e[0..kEv) around its kernels; returns
-  // whether it re-sorted.
-  bool enqueue_step_events(hipEvent_t* e, bool do_sort, const Pool& p) {
-    bool sort = do_sort && sorting() && total_agents_ > 0;
+  // Enqueues absolute step `step` with events e[0..kEv) around its kernels;
+  // returns whether it re-sorted.
+  bool enqueue_step_events(hipEvent_t* e, uint64_t step, const Pool& p) {
+    bool sort = sorts_at(step);
     if (sort) {
       (void)hipEventRecord(e[0], stream);
-      launch_morton_sort(p, agents_[acur_], agents_[acur_ ^ 1], sort_, stream);
+      enqueue_sort(p);
       (void)hipEventRecord(e[1], stream);
-      acur_ ^= 1;
-      tiles_ready_ = true;
     }
     (void)hipEventRecord(e[2], stream);
-    enqueue_agents(p);
+    enqueue_agents(p, step);
     (void)hipEventRecord(e[3], stream);
     launch_trail(p, trail_[cur_], trail_[cur_ ^ 1], stream);
     (void)hipEventRecord(e[4], stream);
@@ -1818,7 +1883,7 @@ class Engine {
     for (uint32_t done = 0; done < n && rc == SLM_OK;) {
       uint32_t m = n - done < batch ? n - done : batch;
       for (uint32_t i = 0; i < m; i++) {
-        sorted[i] = enqueue_step_events(&ev[static_cast<size_t>(i) * kEv], sort_due(steps_done), p);
+        sorted[i] = enqueue_step_events(&ev[static_cast<size_t>(i) * kEv], steps_done, p);
         steps_done++;
       }
       hipError_t err = hipEventSynchronize(ev[static_cast<size_t>(m - 1) * kEv + 4]);
@@ -1883,13 +1948,11 @@ class Engine {
       tc.sorted[j] = sort;
       if (sort) {
         add_event(ev[0]);
-        add_child([&] { launch_morton_sort(p, agents_[acur_], agents_[acur_ ^ 1], sort_, stream); });
+        add_child([&] { enqueue_sort(p); });
         add_event(ev[1]);
-        acur_ ^= 1;
-        tiles_ready_ = true;
       }
       add_event(ev[2]);
-      add_child([&] { enqueue_agents(p); });
+      add_child([&] { enqueue_agents(p, steps_done + j); });
       add_event(ev[3]);
       add_child([&] { launch_trail(p, trail_[cur_], trail_[cur_ ^ 1], stream); });
       add_event(ev[4]);

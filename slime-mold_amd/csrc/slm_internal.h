@@ -84,7 +84,7 @@ struct Instance {
 struct WorkItem {
   uint32_t inst, tile, begin, end;
 };
-constexpr uint32_t kItemAgents = 4096;  // agents per work item at most
+constexpr uint32_t kItemAgents = 4096;  // agents per work item (0.5 to 1.5 times it, where a tile has them)
 
 // A launchable description of a pool, with device copies of its tables.
 struct Pool {
@@ -104,10 +104,8 @@ struct Pool {
   // tiled sensing (valid after a re-sort has built the work list)
   uint32_t total_tiles;
   const uint32_t* tile_inst;   // device: instance of each tile
-  WorkItem* items;             // device: work list, at most max_items entries
-  uint32_t* item_total;        // device: number of valid work items
+  WorkItem* items;             // device: work list, max_items entries, empty ones last
   uint32_t max_items;
-  uint32_t resort_interval;    // steps agents may drift from their tile between re-sorts
   uint32_t agents_per_group;   // agents per workgroup of the global agent pass (k * kAgentBlock)
   uint32_t preload_rows;       // 4, 8 or 16 when every strip instance has tiles of that height, else 0
   int stochastic_rounding;     // bf16 trail-pass stores round stochastically (deterministic hash)
@@ -132,6 +130,54 @@ constexpr uint32_t gauss_th(int storage, int rclass) {
 }
 
 constexpr uint32_t kTileLog2 = 6;  // sensing tiles of 64 x 64 cells
+constexpr uint32_t kTileLds = 81920;  // LDS bytes of a tile's window: two workgroups to a CU
+
+// The margin that a tile's window has around it, `steps` steps after the re-sort:
+// sensors reach sensor_dist * (1 + 2^-22) and a bilinear tap one cell more, a move
+// speed * time step; 3 cells cover the roundings of positions below 2^22.
+struct TileReach {
+  float reach;  // from where an agent stands
+  float move;   // a step's move at most
+  int margin;   // reach and drift, whole cells (1027 at most)
+};
+__host__ __device__ inline TileReach tile_reach(const DevParams& p, uint32_t steps) {
+  const float vmin = __builtin_fabsf(p.speed_min), vmax = __builtin_fabsf(p.speed_max);
+  const float sd = __builtin_fabsf(p.sensor_dist);
+  TileReach r;
+  r.move = (vmin > vmax ? vmin : vmax) * 0.016f;
+  r.reach = (sd > r.move ? sd : r.move) + 3.0f;
+  const float m = r.reach + r.move * static_cast<float>(steps);
+  r.margin = static_cast<int>(__builtin_ceilf(m < 1024.0f ? m : 1024.0f));
+  return r;
+}
+// 16-byte chunks per row (V cells each) and rows of the window of the tile at
+// (tx, ty), and its first cell.  An odd number of chunks, so that LDS rows start
+// on other banks.
+struct TileExtent {
+  int x0, y0, cpr, rows;
+};
+__host__ __device__ inline TileExtent tile_extent(const Instance& in, int tx, int ty, int margin,
+                                                  int V) {
+  const int tile = 1 << in.tile_log2;
+  const int W = static_cast<int>(in.width), H = static_cast<int>(in.height);
+  TileExtent e;
+  e.x0 = tx - margin > 0 ? tx - margin : 0;
+  if (W % V == 0) e.x0 -= e.x0 % V;  // aligned chunks where rows are whole chunks
+  e.y0 = ty - margin > 0 ? ty - margin : 0;
+  const int x1 = tx + tile + margin < W ? tx + tile + margin : W;
+  const int y1 = ty + tile + margin < H ? ty + tile + margin : H;
+  e.cpr = ((x1 - e.x0 + V - 1) / V) | 1;
+  e.rows = y1 - e.y0;
+  return e;
+}
+// Whether it can be staged: it fits the LDS (as f32), its chunk indexes divide
+// exactly (rows <= 1024), and the trail has 32-bit byte offsets.
+__host__ __device__ inline bool tile_staged(const Instance& in, const TileExtent& e, int V) {
+  const uint32_t bytes = 16u / static_cast<uint32_t>(V);
+  return in.width < (1u << 24) / bytes &&
+         static_cast<uint64_t>(in.width) * in.height < (1ull << 32) / bytes && e.rows <= 1024 &&
+         e.cpr <= 64 && static_cast<uint32_t>(e.cpr * e.rows * V * 4) <= kTileLds;
+}
 
 constexpr int kAgentBlock = 256;
 constexpr int kTrailBlock = 256;
@@ -144,6 +190,15 @@ __device__ inline uint32_t xcd_logical_block(uint32_t b, uint32_t nb) {
   uint32_t xcd = b & 7u, idx = b >> 3;
   uint32_t per = nb >> 3, rem = nb & 7u;
   return xcd < rem ? xcd * (per + 1u) + idx : rem * (per + 1u) + (xcd - rem) * per + idx;
+}
+
+// The block that xcd_logical_block gives logical block k.
+__device__ inline uint32_t xcd_block_of(uint32_t k, uint32_t nb) {
+  uint32_t per = nb >> 3, rem = nb & 7u;
+  uint32_t head = rem * (per + 1u);  // logical blocks of the first rem XCDs
+  uint32_t xcd = k < head ? k / (per + 1u) : rem + (k - head) / per;
+  uint32_t idx = k < head ? k % (per + 1u) : (k - head) % per;
+  return idx * 8u + xcd;
 }
 
 // ---- persistent launches -------------------------------------------------------
@@ -236,11 +291,10 @@ void plan_tiles(Instance& in, uint32_t cell_log2, uint32_t tile_log2);
 // ---- launchers (all asynchronous on `stream`) ----------------------------
 void launch_agents(const Pool& pool, const AgentSoA& a, void* trail, hipStream_t stream);
 // The same update with each tile's trail window staged in LDS (needs the work
-// list of the latest re-sort); bit-identical to launch_agents.
-void launch_agents_tiled(const Pool& pool, const AgentSoA& a, void* trail, hipStream_t stream);
-// LDS bytes the tiled pass stages per workgroup for this storage format.
-constexpr uint32_t kWindowBytes = 65536;
-uint32_t window_side(int storage);
+// list of the latest re-sort); bit-identical to launch_agents.  drift_steps: the
+// steps since that re-sort, this one included.
+void launch_agents_tiled(const Pool& pool, const AgentSoA& a, void* trail, uint32_t drift_steps,
+                         hipStream_t stream);
 void launch_trail(const Pool& pool, const void* trail_in, void* trail_out, hipStream_t stream);
 void launch_set_params(DevParams* dst, const DevParams& src, hipStream_t stream);
 void launch_init_agents(const Instance& in, const AgentSoA& a, int pos64, uint64_t seed,

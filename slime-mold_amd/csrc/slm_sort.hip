@@ -314,37 +314,58 @@ __global__ __launch_bounds__(kAgentBlock) void canonical_copy_kernel(
   if (dst.id) dst.id[d] = local;
 }
 
-// Work items of each tile: ceil(agents / kItemAgents), 0 for an empty tile.
+// Work items of a tile of n agents, cut into equal parts of about kItemAgents.
+__device__ inline uint32_t items_of(uint32_t n) {
+  return n == 0u ? 0u : max(1u, (n + kItemAgents / 2u) / kItemAgents);
+}
+
+// Work items of each tile, 0 for an empty one.
 __global__ void tile_count_kernel(const Instance* insts, const uint32_t* tile_inst,
                                   uint32_t ntiles, uint32_t cell_log2, const uint32_t* offset,
-                                  uint32_t* tile_items) {
+                                  uint32_t* tile_items, WorkItem* items, uint32_t max_items) {
   uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
+  // every entry starts empty; tile_items_kernel fills those there are
+  for (uint32_t i = g; i < max_items; i += gridDim.x * blockDim.x) items[i] = WorkItem{0, 0, 0, 0};
   if (g >= ntiles) return;
   const Instance in = insts[tile_inst[g]];
   uint32_t t = g - in.tile_off;
   uint32_t per = 1u << (2u * (in.tile_log2 - cell_log2));  // bins per tile
   uint32_t b0 = in.bin_off + t * per;
   uint32_t n = offset[b0 + per] - offset[b0];
-  tile_items[g] = (n + kItemAgents - 1u) / kItemAgents;
+  tile_items[g] = items_of(n);
 }
 
-// Writes each tile's work items at its scanned offset; the last tile also
-// writes the total.
+// Writes each tile's work items.  Item k of the list goes to the entry of the
+// block that takes logical block k of a launch over the items there are, so
+// that every XCD works on one contiguous run of tiles and none is left without:
+// a map over the whole list, whose empty end the last XCDs would get, left
+// three of the eight idle.
 __global__ void tile_items_kernel(const Instance* insts, const uint32_t* tile_inst,
                                   uint32_t ntiles, uint32_t cell_log2, const uint32_t* offset,
-                                  const uint32_t* item_off, WorkItem* items, uint32_t* total) {
+                                  const uint32_t* item_off, int xcd_remap, WorkItem* items) {
   uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
   if (g >= ntiles) return;
-  uint32_t ii = tile_inst[g];
-  const Instance in = insts[ii];
-  uint32_t t = g - in.tile_off;
-  uint32_t per = 1u << (2u * (in.tile_log2 - cell_log2));
-  uint32_t b0 = in.bin_off + t * per;
-  uint32_t begin = offset[b0], end = offset[b0 + per];
-  uint32_t at = item_off[g];
-  for (uint32_t s = begin; s < end; s += kItemAgents)
-    items[at++] = WorkItem{ii, t, s, min(s + kItemAgents, end)};
-  if (g == ntiles - 1u) *total = at;
+  auto range = [&](uint32_t tile, uint32_t& ii, uint32_t& t, uint32_t& begin, uint32_t& end) {
+    ii = tile_inst[tile];
+    const Instance in = insts[ii];
+    t = tile - in.tile_off;
+    uint32_t per = 1u << (2u * (in.tile_log2 - cell_log2));
+    uint32_t b0 = in.bin_off + t * per;
+    begin = offset[b0];
+    end = offset[b0 + per];
+  };
+  uint32_t ii, t, begin, end;
+  range(ntiles - 1u, ii, t, begin, end);
+  const uint32_t total = item_off[ntiles - 1u] + items_of(end - begin);
+  range(g, ii, t, begin, end);
+  const uint32_t n = items_of(end - begin);
+  auto cut = [&](uint32_t i) {
+    return begin + static_cast<uint32_t>(static_cast<uint64_t>(end - begin) * i / n);
+  };
+  for (uint32_t i = 0; i < n; i++) {
+    const uint32_t k = item_off[g] + i;
+    items[xcd_remap ? xcd_block_of(k, total) : k] = WorkItem{ii, t, cut(i), cut(i + 1u)};
+  }
 }
 
 inline uint32_t next_pow2(uint32_t v) {
@@ -415,11 +436,12 @@ void launch_morton_sort(const Pool& pool, const AgentSoA& src, const AgentSoA& d
   if (pool.items) {  // work list of the tiled agent pass
     uint32_t nt = pool.total_tiles;
     tile_count_kernel<<<blocks_for(nt, 256), 256, 0, stream>>>(
-        pool.inst, pool.tile_inst, nt, pool.sort_cell_log2, s.offset, s.tile_items);
+        pool.inst, pool.tile_inst, nt, pool.sort_cell_log2, s.offset, s.tile_items, pool.items,
+        pool.max_items);
     scan(s, s.tile_items, nt, s.tile_items, 0, stream);
     tile_items_kernel<<<blocks_for(nt, 256), 256, 0, stream>>>(
-        pool.inst, pool.tile_inst, nt, pool.sort_cell_log2, s.offset, s.tile_items, pool.items,
-        pool.item_total);
+        pool.inst, pool.tile_inst, nt, pool.sort_cell_log2, s.offset, s.tile_items,
+        pool.xcd_remap, pool.items);
   }
 }
 

@@ -182,6 +182,96 @@ SLM_TRIG_FN void slm_sincosf_finite(float x, float* s_out, float* c_out) {
   *c_out = cs;
 }
 
+/*
+ * sin and cos of |x| < SLM_TRIG_SMALL_MAX, the bits of slm_sincosf_finite in
+ * fewer issue cycles.  On gfx950 a VALU multiply, add, fma, and/xor/bitop3 or
+ * 32-bit add issues in half the cycles of a compare, a select, a rounding or a
+ * conversion (measured 2.3 against 4.4 cycles per wave), so
+ *   - k = rint(ax * 2/pi) is an add and a subtract of 1.5 * 2^23: the sum's
+ *     ulp is 1 and its rounding is to nearest even, as rint's, and the low two
+ *     bits of its representation are those of k (1.5 * 2^23 is a multiple of 4);
+ *   - the quadrant's swap of sin and cos and the signs are bit operations.
+ * The three constants that instructions take with |x| or as a third operand,
+ * where no literal fits, are arguments: 2/pi, C1 and the sign bit, which GPU
+ * callers keep in vector registers (a scalar register operand halves the rate).
+ */
+#define SLM_RINT_MAGIC 12582912.0f /* 1.5 * 2^23 */
+SLM_TRIG_FN void slm_sincosf_small_k(float x, float two_over_pi, float c1, uint32_t sign,
+                                     float* s_out, float* c_out) {
+  uint32_t ux = slm_f32_bits(x);
+  float ax = __builtin_fabsf(x);
+  float t = ax * two_over_pi;
+  t = t + SLM_RINT_MAGIC;
+  uint32_t q = slm_f32_bits(t);
+  float k = t - SLM_RINT_MAGIC;
+  float r = __builtin_fmaf(-k, c1, ax);
+  r = __builtin_fmaf(-k, SLM_PIO2_C2, r);
+  r = __builtin_fmaf(-k, SLM_PIO2_C3, r);
+  float r2 = r * r;
+  float ps = __builtin_fmaf(r2, SLM_SIN_T4, SLM_SIN_T3);
+  ps = __builtin_fmaf(r2, ps, SLM_SIN_T2);
+  ps = __builtin_fmaf(r2, ps, SLM_SIN_T1);
+  float r3 = r * r2;
+  uint32_t s = slm_f32_bits(__builtin_fmaf(r3, ps, r));
+  float pc = __builtin_fmaf(r2, SLM_COS_T5, SLM_COS_T4);
+  pc = __builtin_fmaf(r2, pc, SLM_COS_T3);
+  pc = __builtin_fmaf(r2, pc, SLM_COS_T2);
+  pc = __builtin_fmaf(r2, pc, SLM_COS_T1);
+  uint32_t c = slm_f32_bits(__builtin_fmaf(r2, pc, 1.0f));
+  uint32_t swap = (s ^ c) & (0u - (q & 1u));
+  uint32_t h = q << 30; /* the quadrant's bits at 31 and 30 */
+  *s_out = slm_f32_from_bits(s ^ swap ^ ((h ^ ux) & sign));
+  *c_out = slm_f32_from_bits(c ^ swap ^ ((h + 0x40000000u) & sign));
+}
+SLM_TRIG_FN void slm_sincosf_small(float x, float* s_out, float* c_out) {
+  slm_sincosf_small_k(x, SLM_TWO_OVER_PI_F, SLM_PIO2_C1, 0x80000000u, s_out, c_out);
+}
+
+/*
+ * sin of SLM_TRIG_SMALL_MAX <= |x| < 2^32, the bits of slm_sincosf_finite: the
+ * jitter hash's range below 3.3e8 agents.  The same Payne-Hanek product; the
+ * window's start p is 19..38 here, so 2/pi's bits from extended position 7 on,
+ * as four fixed words, give every window with one funnel shift of 12..31 bits
+ * per word and no selects.
+ */
+#define SLM_2OPI_U0 (SLM_2OPI_W1 >> 25)
+#define SLM_2OPI_U1 ((SLM_2OPI_W1 << 7) | (SLM_2OPI_W2 >> 25))
+#define SLM_2OPI_U2 ((SLM_2OPI_W2 << 7) | (SLM_2OPI_W3 >> 25))
+#define SLM_2OPI_U3 ((SLM_2OPI_W3 << 7) | (SLM_2OPI_W4 >> 25))
+#define SLM_TRIG_MID_MAX 4294967296.0f
+SLM_TRIG_FN float slm_sinf_mid(float x) {
+  uint32_t ux = slm_f32_bits(x);
+  uint32_t e = (ux >> 23) & 0xffu;
+  uint64_t m = (ux & 0x7fffffu) | 0x800000u;
+  int s = (int)e - 127; /* p - 7 with p = e - 150 + 30; 12..31 */
+  uint64_t hi = slm_funnel32(SLM_2OPI_U0, SLM_2OPI_U1, s);
+  uint64_t mid = slm_funnel32(SLM_2OPI_U1, SLM_2OPI_U2, s);
+  uint64_t lo = slm_funnel32(SLM_2OPI_U2, SLM_2OPI_U3, s);
+  uint64_t acc = m * lo;
+  acc = (acc >> 32) + m * mid;
+  uint32_t w1 = (uint32_t)acc;
+  acc = (acc >> 32) + m * hi;
+  uint64_t top = (acc << 32) | w1; /* 2 integer bits, 62 fraction bits */
+  /* the nearest multiple of pi/2 and the signed rest */
+  uint32_t q = (uint32_t)((top + ((uint64_t)1 << 61)) >> 62);
+  int64_t frac = (int64_t)(top << 2) >> 2;
+  int64_t f53 = frac / 512;
+  float r = (float)((double)f53 * SLM_PIO2_X2M53_D);
+  float r2 = r * r;
+  float ps = __builtin_fmaf(r2, SLM_SIN_T4, SLM_SIN_T3);
+  ps = __builtin_fmaf(r2, ps, SLM_SIN_T2);
+  ps = __builtin_fmaf(r2, ps, SLM_SIN_T1);
+  float r3 = r * r2;
+  uint32_t sn = slm_f32_bits(__builtin_fmaf(r3, ps, r));
+  float pc = __builtin_fmaf(r2, SLM_COS_T5, SLM_COS_T4);
+  pc = __builtin_fmaf(r2, pc, SLM_COS_T3);
+  pc = __builtin_fmaf(r2, pc, SLM_COS_T2);
+  pc = __builtin_fmaf(r2, pc, SLM_COS_T1);
+  uint32_t c = slm_f32_bits(__builtin_fmaf(r2, pc, 1.0f));
+  uint32_t swap = (sn ^ c) & (0u - (q & 1u));
+  return slm_f32_from_bits(sn ^ swap ^ (((q << 30) ^ ux) & 0x80000000u));
+}
+
 /* sin and cos of one float argument; NaN for NaN or infinity. */
 SLM_TRIG_FN void slm_sincosf(float x, float* s_out, float* c_out) {
   if (!(__builtin_fabsf(x) <= 3.4028234663852886e38f)) { /* NaN or infinity */
