@@ -254,7 +254,7 @@ __device__ inline void finish_row(float (&t)[Codec<S>::kVec + 2], const RawRow<S
 constexpr int kAhead = 4;
 
 template <int S, int M>
-__device__ inline void strip_unit(const typename Codec<S>::elem* in, typename Codec<S>::elem* out,
+__device__ __forceinline__ void strip_unit(const typename Codec<S>::elem* in, typename Codec<S>::elem* out,
                                   const Instance& inst, const DevParams& p, uint32_t tile,
                                   uint32_t lane, int streaming) {
   const bool nt_load = (streaming & kStreamLoads) != 0;
@@ -334,7 +334,7 @@ __device__ inline void strip_unit(const typename Codec<S>::elem* in, typename Co
 // re-read fewer halo rows (R + 2 loads per R rows) without losing the memory
 // parallelism that short tiles get from having more waves.
 template <int S, int M, int R>
-__device__ inline void strip_unit_preload(const typename Codec<S>::elem* in,
+__device__ __forceinline__ void strip_unit_preload(const typename Codec<S>::elem* in,
                                           typename Codec<S>::elem* out, const Instance& inst,
                                           const DevParams& p, uint32_t tile, uint32_t lane,
                                           int streaming) {
@@ -401,7 +401,7 @@ __device__ inline void strip_unit_preload(const typename Codec<S>::elem* in,
 // R = 0: streaming strip units of any height; R = 4, 8 or 16: every strip
 // instance of the launch has R-row tiles, loaded whole.
 template <int S, int M, int R>
-__device__ inline void strip_dispatch(const typename Codec<S>::elem* in,
+__device__ __forceinline__ void strip_dispatch(const typename Codec<S>::elem* in,
                                       typename Codec<S>::elem* out, const Instance& inst,
                                       const DevParams& p, uint32_t tile, uint32_t lane,
                                       int streaming) {
@@ -413,7 +413,7 @@ __device__ inline void strip_dispatch(const typename Codec<S>::elem* in,
 
 // One 64-cell unit, one cell per lane, any row length.
 template <int S>
-__device__ inline void cell_unit(const typename Codec<S>::elem* in, typename Codec<S>::elem* out,
+__device__ __forceinline__ void cell_unit(const typename Codec<S>::elem* in, typename Codec<S>::elem* out,
                                  const Instance& inst, const DevParams& p, uint32_t unit,
                                  uint32_t lane) {
   const uint32_t w = inst.width, h = inst.height;
@@ -451,7 +451,7 @@ struct TrailArgs {
 
 // One logical workgroup `blk` (kTrailWavesPerBlock wave units) of the pass.
 template <int S, int R>
-__device__ inline void trail_block(const TrailArgs& a, const Instance* __restrict__ insts,
+__device__ __forceinline__ void trail_block(const TrailArgs& a, const Instance* __restrict__ insts,
                                    const DevParams* __restrict__ params,
                                    const uint32_t* __restrict__ block_inst, uint32_t blk) {
   using elem = typename Codec<S>::elem;
@@ -477,19 +477,25 @@ __device__ inline void trail_block(const TrailArgs& a, const Instance* __restric
 }
 
 // Tables as restrict arguments: their wave-uniform loads become scalar loads.
-// With a.claim set the launch is persistent (persistent_blocks).
-template <int S, int R>
+// kClaim: a persistent launch (persistent_blocks, a.claim set), a kernel of its own
+// so that each holds one copy of the body: 62 VGPRs (8 waves per SIMD) against 69
+// with 4-row tiles of 16-bit cells.  The body is forced inline: the compiler called
+// the 16-row tiles of 16-bit cells as a function otherwise (245 VGPRs and a stack,
+// now 136), which took 113 us at 8192^2 bf16 with stochastic rounding and 106 us
+// without; now 62 and 53 us.
+template <int S, int R, bool kClaim>
 __global__ __launch_bounds__(kTrailBlock) void trail_kernel(
     TrailArgs a, const Instance* __restrict__ insts, const DevParams* __restrict__ params,
     const uint32_t* __restrict__ block_inst) {
-  __shared__ uint32_t s_claim;
-  if (!a.claim) {
-    uint32_t blk = a.xcd_remap ? xcd_logical_block(blockIdx.x, gridDim.x) : blockIdx.x;
-    trail_block<S, R>(a, insts, params, block_inst, blk);
-    return;
+  if constexpr (kClaim) {
+    __shared__ uint32_t s_claim;
+    persistent_blocks(a.claim, a.blocks, &s_claim, [&](uint32_t blk) {
+      trail_block<S, R>(a, insts, params, block_inst, blk);
+    });
+  } else {
+    trail_block<S, R>(a, insts, params, block_inst,
+                      a.xcd_remap ? xcd_logical_block(blockIdx.x, gridDim.x) : blockIdx.x);
   }
-  persistent_blocks(a.claim, a.blocks, &s_claim,
-                    [&](uint32_t blk) { trail_block<S, R>(a, insts, params, block_inst, blk); });
 }
 
 __global__ void set_params_kernel(DevParams* dst, DevParams src) { *dst = src; }
@@ -634,20 +640,22 @@ void launch_trail_t(const Pool& pool, const void* in, void* out, hipStream_t str
   const uint32_t nb = blocks_for(pool.total_units, kTrailWavesPerBlock);
   TrailArgs a{in,         out,         pool.inst,      pool.params, pool.unit_block_inst,
               pool.count, pool.total_units, pool.xcd_remap, pool.streaming, pool.claim_trail, nb};
-  auto go = [&](auto* kernel) {
-    const uint32_t grid = a.claim ? persistent_grid(kernel, nb, kTrailBlock) : nb;
-    kernel<<<grid, kTrailBlock, 0, stream>>>(a, a.inst, a.params, a.block_inst);
+  auto go = [&](auto* direct, auto* persistent) {
+    if (a.claim)
+      persistent<<<persistent_grid(persistent, nb, kTrailBlock), kTrailBlock, 0, stream>>>(
+          a, a.inst, a.params, a.block_inst);
+    else
+      direct<<<nb, kTrailBlock, 0, stream>>>(a, a.inst, a.params, a.block_inst);
   };
   if (pool.preload_rows == 4)
-    go(trail_kernel<S, 4>);
+    go(trail_kernel<S, 4, false>, trail_kernel<S, 4, true>);
   else if (pool.preload_rows == 8)
-    go(trail_kernel<S, 8>);
+    go(trail_kernel<S, 8, false>, trail_kernel<S, 8, true>);
   else if (pool.preload_rows == 16)
-    go(trail_kernel<S, 16>);
+    go(trail_kernel<S, 16, false>, trail_kernel<S, 16, true>);
   else
-    go(trail_kernel<S, 0>);
+    go(trail_kernel<S, 0, false>, trail_kernel<S, 0, true>);
 }
-
 
 // ---- Gaussian diffuse (SLM_FLAG_GAUSSIAN_DIFFUSE) ------------------------------
 // One 256-thread workgroup per tile of kGaussTW x gauss_th(storage) cells.  The tile's
@@ -1133,10 +1141,10 @@ void launch_render(const RenderArgs& args, const LutBytes& lut, int storage, hip
 void prime_persistent_trail() {
   auto each = [](auto s_tag) {
     constexpr int S = decltype(s_tag)::value;
-    (void)persistent_grid(trail_kernel<S, 0>, 8, kTrailBlock);
-    (void)persistent_grid(trail_kernel<S, 4>, 8, kTrailBlock);
-    (void)persistent_grid(trail_kernel<S, 8>, 8, kTrailBlock);
-    (void)persistent_grid(trail_kernel<S, 16>, 8, kTrailBlock);
+    (void)persistent_grid(trail_kernel<S, 0, true>, 8, kTrailBlock);
+    (void)persistent_grid(trail_kernel<S, 4, true>, 8, kTrailBlock);
+    (void)persistent_grid(trail_kernel<S, 8, true>, 8, kTrailBlock);
+    (void)persistent_grid(trail_kernel<S, 16, true>, 8, kTrailBlock);
   };
   each(std::integral_constant<int, SLM_STORAGE_F32>{});
   each(std::integral_constant<int, SLM_STORAGE_BF16>{});
