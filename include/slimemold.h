@@ -325,8 +325,8 @@ typedef struct slm_tuning {
   uint32_t agents_per_group; /* agents one workgroup of the agent pass updates:
                                 256, 512, 1024, 2048 or 4096 */
   uint32_t trail_rows;       /* rows of one trail-pass tile (64*vector-width
-                                columns): 4, 8, 16, 32 or 64; 0 = chosen from the
-                                grid so the launch has >= 8192 waves */
+                                columns): 4, 8, 16, 32 or 64; 0 = the library's
+                                choice (4) */
   uint32_t tiled_sensing;    /* 1 = SLM_FLAG_TILED_SENSING (needs re-sorting),
                                 2 = SLM_FLAG_WINDOW_SENSING, 0 = the library's
                                 choice of global memory or tile windows */

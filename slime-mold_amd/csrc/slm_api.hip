@@ -91,7 +91,6 @@ constexpr uint64_t kMaxAgents = 0xffffff00ull;    // u32 slot index, whole block
 constexpr float kMaxSensorDistance = 4194304.0f;  // keeps sensor taps inside i32
 constexpr uint64_t kMaxTotalBins = 1ull << 30;
 constexpr float kMaxTrailValue = 0x1p100f;        // keeps every 3x3 window sum finite
-constexpr uint32_t kTargetWaves = 8192;           // trail-pass units per pool
 constexpr uint32_t kKnownFlags = SLM_FLAG_NO_XCD_REMAP | SLM_FLAG_F64_POSITIONS |
                                  SLM_FLAG_TILED_SENSING | SLM_FLAG_STOCHASTIC_ROUNDING |
                                  SLM_FLAG_GAUSSIAN_DIFFUSE | SLM_FLAG_WINDOW_SENSING |
@@ -1357,9 +1356,7 @@ class Engine {
     uint64_t units = 0, bins = 0;
     for (size_t k = 0; k < spec.size(); k++) {
       Instance& in = inst[k];
-      uint32_t target = static_cast<uint32_t>(
-          std::max<uint64_t>(1, kTargetWaves * cells(k) / std::max<uint64_t>(1, total_cells)));
-      plan_trail(in, cfg.storage, target, cfg.trail_rows);
+      plan_trail(in, cfg.storage, cfg.trail_rows);
       in.unit_off = static_cast<uint32_t>(units);
       units += in.units;
       uint32_t cl = cfg.sort_cell_log2;

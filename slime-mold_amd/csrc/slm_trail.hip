@@ -987,16 +987,18 @@ void launch_gauss_t(const Pool& pool, const void* in, void* out, hipStream_t str
 
 }  // namespace
 
-void plan_trail(Instance& in, int storage, uint32_t target_waves, uint32_t fixed_rows) {
+void plan_trail(Instance& in, int storage, uint32_t fixed_rows) {
   uint32_t v = storage == SLM_STORAGE_F32 ? 4u : 8u;
   if (in.width >= v) {
     in.ntx = (in.width + 64u * v - 1u) / (64u * v);
-    // rows per strip unit: fixed, or the longest of 64..4 that still gives
-    // target_waves units
-    uint32_t rows = fixed_rows ? fixed_rows : 64u;
-    while (!fixed_rows && rows > 4 &&
-           static_cast<uint64_t>(in.ntx) * ((in.height + rows - 1) / rows) < target_waves)
-      rows >>= 1;
+    // Rows per strip unit: fixed, or 4.  The shortest tiles are loaded whole, keep the
+    // most waves, and their halo rows are found in the L2: at every size they take
+    // the least time, or within 2% of it, in us, 4 / 8 / 16 / 64 rows:
+    //   1024^2 f32 7.0 / 8.4 / 11.2 / 36    4096^2 f32 21.8 / 23.0 / 23.1 / 41
+    //   8192^2 f32 102 / 107 / 107 / 118    8192^2 bf16 46.8 / 45.9 / 51.9 / 55.5
+    // (taller tiles on larger grids, for at least 8192 waves, gave the last a 64-row
+    // tile in f32 and a 16-row one in bf16)
+    const uint32_t rows = fixed_rows ? fixed_rows : 4u;
     in.tile_rows = rows;
     in.units = in.ntx * ((in.height + rows - 1u) / rows);
   } else {
