@@ -55,7 +55,8 @@ struct TrailRead<SLM_STORAGE_F32> {
   }
   __device__ static void mark(void* t, uint32_t i) {
     uint32_t* p = static_cast<uint32_t*>(t) + i;
-    *p = *p | 0x80000000u;
+    const uint32_t v = *p;
+    if (!(v >> 31)) *p = v | 0x80000000u;
   }
 };
 
@@ -66,10 +67,14 @@ __device__ inline uint32_t load_u16_pair(const void* t, uint32_t i) {
 }
 
 // 16-bit cells are marked with a 2-byte store, which leaves the neighbour in
-// the same 32-bit word untouched.
+// the same 32-bit word untouched.  A cell that is marked already is not stored
+// again: without a re-sort the agents of all XCDs store into all lines, and these
+// stores, several to a cell where trails form, bound the pass (1365 x 767 f32, never
+// re-sorted, 3 * 10^6 agents: 274 -> 167 us; re-sorted pools gain up to 2%).
 __device__ inline void mark16(void* t, uint32_t i) {
   uint16_t* p = static_cast<uint16_t*>(t) + i;
-  *p = static_cast<uint16_t>(*p | 0x8000u);
+  const uint32_t v = *p;
+  if (!(v & 0x8000u)) *p = static_cast<uint16_t>(v | 0x8000u);
 }
 
 template <>
@@ -647,9 +652,9 @@ __global__ __launch_bounds__(kAgentBlock) void agents_kernel(
 // The LDS reads the same pairs at 64 banks a cycle, and the window comes in
 // coalesced, 16 bytes a lane: 4.4 cells an agent at one agent a cell.  What it
 // measured, us per pass with the global pass's in brackets: 4096^2 f32 with 2^24
-// agents 180 (275) while trails form, 159 (205) once formed; 1600 x 900 with
+// agents 175 (275) while trails form, 155 (205) once formed; 1600 x 900 with
 // 10^7 agents 96 (137) and 78 (109); 8192^2 bf16 with f64 positions and 2^26
-// agents 890 to 915 (1030 to 1200).
+// agents 814 to 900 (1030 to 1200).
 //
 // Shape, all measured: 64-cell tiles and 1024 threads, two workgroups to a CU
 // (80 KiB of LDS each, 64 VGPRs), so that one computes while the other stages;
@@ -673,10 +678,20 @@ __global__ __launch_bounds__(kAgentBlock) void agents_kernel(
 // keeps its own form: it gains nothing from fewer instructions.)
 // A cell's mark in two halves, the load of the 16 bits that hold its sign and
 // their store, so that a caller can have other stores between them.
+// A mark from the window is noted there too (the upper half of the f32 cell, which
+// the taps read as |T|), so that the tile's later agents skip the cell: 4096^2 f32
+// with 2^24 agents 169 -> 164 us per pass, 8192^2 bf16 with f64 positions 826 -> 814.
 struct Mark {
   uint16_t* p;
   uint32_t raw;
-  __device__ void store() const { *p = static_cast<uint16_t>(raw | 0x8000u); }
+  uint16_t* win;   // in the window, or nullptr
+  uint32_t upper;  // what `win` holds
+  __device__ void store() const {
+    if (!(raw & 0x8000u)) {
+      *p = static_cast<uint16_t>(raw | 0x8000u);
+      if (win) *win = static_cast<uint16_t>(upper | 0x8000u);
+    }
+  }
 };
 
 // Whether cells (x0, y0) .. (x0 + 1, y0 + 1) lie in the grid: a negative
@@ -729,7 +744,7 @@ struct TileTaps {
   }
   __device__ Mark mark(uint32_t x, uint32_t y) const {
     uint16_t* p = half_cell(x, y);
-    return {p, *p};
+    return {p, *p, nullptr, 0u};
   }
   // The cell's |T| is in the window: the mark needs no load from the trail.
   // (Marking in the window and storing the marked cells a row per wave at the
@@ -742,7 +757,8 @@ struct TileTaps {
                                static_cast<_Float16>(*reinterpret_cast<const float*>(p)));
     else
       raw = *reinterpret_cast<const uint16_t*>(p + 2);
-    return {half_cell(x, y), raw};
+    uint16_t* u = reinterpret_cast<uint16_t*>(const_cast<char*>(p) + 2);
+    return {half_cell(x, y), raw, u, *u};
   }
   // The 16 bits that hold a cell's sign, in a trail below 2^32 bytes with rows
   // below 2^24 (tile_staged).
