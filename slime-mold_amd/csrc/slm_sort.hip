@@ -10,6 +10,8 @@
 // which is harmless: an agent's update depends only on its own state, its
 // original index and the step-start trail, and the deposit marks commute, so
 // any permutation gives the same result.
+#include <type_traits>
+
 #include "slm_internal.h"
 
 namespace slm {
@@ -65,143 +67,150 @@ __global__ void zero_u32_kernel(uint32_t* p, uint32_t n) {
   if (i < n) p[i] = 0u;
 }
 
-// Bins each agent and takes its rank inside the bin, with as few global
-// atomics as possible: agents re-sorted earlier arrive grouped by bin, so a
-// block's agents usually span a handful of consecutive bins.  Each agent takes
-// its rank in the block from an LDS atomic on its bin's counter, and one
-// global atomic per distinct bin of the block reserves the block's range.
-// (Dense instances put ~10^4 agents in one bin; a global atomic per wave and
-// bin serialised ~10^2 times more.)  Blocks whose bins span a wider range fall
-// back to one global atomic per wave and bin.  Ranks are not in a fixed order.
-//
-// A block bins kCountPer x 256 agents, each thread kCountPer of them (slots
-// q*256 + threadIdx.x of the block's range), all loaded before any is used:
-// the kernel is a chain of load -> barrier -> global atomic -> barrier per
-// block, and with one agent per thread that latency, not bandwidth, set its
-// time.
-constexpr uint32_t kLocalBins = 2048;
-constexpr int kCountPer = 4;
-constexpr uint32_t kCountSlots = kCountPer * kAgentBlock;
+// A workgroup of the count and scatter kernels takes kSortPer x 256 consecutive
+// slots, each thread kSortPer of them (slots q*256 + threadIdx.x of the range).
+// Agents re-sorted earlier arrive grouped by bin, so these usually stand in a few
+// neighbouring bins, which the workgroup counts in LDS: one global atomic per
+// distinct bin of the workgroup.  (Dense instances put ~10^4 agents in one bin; a
+// global atomic per wave and bin serialised ~10^2 times more.)  A bin's entry there
+// is its key mod kLocalBins: the Morton codes of any 32 x 32 bins differ in their low
+// 10 bits, also where the region straddles an edge of a large aligned square and
+// its codes lie far apart (a table by distance from the lowest code refuses those,
+// a quarter of the workgroups or more).  Where two bins meet in an entry the
+// workgroup falls back to atomics on the global counters.
+constexpr uint32_t kLocalBins = 1024;  // LDS for 5 workgroups a CU (2048: 4, up to 7% slower)
+constexpr int kSortPer = 4;
+constexpr uint32_t kSortSlots = kSortPer * kAgentBlock;
 
-__global__ __launch_bounds__(kAgentBlock) void count_kernel(
-    AgentSoA a, const Instance* insts, const DevParams* params, const uint32_t* block_inst,
-    uint32_t ninst, uint32_t total, int pos64, uint32_t cell_log2, uint32_t sort_key,
-    int xcd_remap, uint32_t* rank, uint32_t* count) {
-  __shared__ uint32_t s_min, s_max;
-  __shared__ uint32_t s_cnt[kLocalBins];
-  __shared__ uint32_t s_base[kLocalBins];
-  // XCD-contiguous blocks, as in the scatter: neighbouring slots, their bins'
-  // counters and their output ranges stay with one XCD's L2 (the re-sort of
-  // the 256-instance mix measured 10% faster)
-  const uint32_t base =
-      (xcd_remap ? xcd_logical_block(blockIdx.x, gridDim.x) : blockIdx.x) * kCountSlots;
-  uint32_t k[kCountPer];
-  bool act[kCountPer];
-  float px[kCountPer], py[kCountPer], pth[kCountPer];
-  // the heading only enters refined keys: the plain key loads positions only
-  const bool heading = sort_key != 0u;
+// The tables of a re-sort kernel's launch.
+struct SortArgs {
+  const Instance* insts;
+  const DevParams* params;
+  const uint32_t* block_inst;  // per kAgentBlock slots
+  uint32_t ninst, total, cell_log2, sort_key;
+  int xcd_remap;
+};
+
+// XCD-contiguous workgroups: neighbouring slots, their bins' counters and their
+// output ranges stay with one XCD's L2 (the re-sort of the 256-instance mix
+// measured 10% faster).
+__device__ inline uint32_t sort_base(const SortArgs& g) {
+  return (g.xcd_remap ? xcd_logical_block(blockIdx.x, gridDim.x) : blockIdx.x) * kSortSlots;
+}
+
+// Slot q of this thread, and whether there is one (a 64-bit test: near the 2^32 - 256
+// agent limit the last workgroup's slots wrap).
+__device__ inline bool sort_slot(const SortArgs& g, uint32_t base, int q, uint32_t& j) {
+  j = base + q * kAgentBlock + threadIdx.x;
+  return uint64_t(base) + q * kAgentBlock + threadIdx.x < g.total;
+}
+
+// The keys of the workgroup's agents, their ranks among its agents of the bin, and
+// whether each bin has an entry of its own in `s_cnt`, which then holds the bin's
+// agents (uniform).  s_tag is scratch, free again on return.
+struct Keys {
+  uint32_t k[kSortPer], r[kSortPer];
+  bool act[kSortPer];
+  bool local;
+  __device__ uint32_t entry(int q) const { return k[q] & (kLocalBins - 1u); }
+};
+__device__ inline Keys block_keys(const SortArgs& g, uint32_t base, const float (&x)[kSortPer],
+                                  const float (&y)[kSortPer], const float (&th)[kSortPer],
+                                  uint32_t* s_cnt, uint32_t* s_tag) {
+  for (uint32_t i = threadIdx.x; i < kLocalBins; i += kAgentBlock) s_cnt[i] = 0u;
+  Keys t;
 #pragma unroll
-  for (int q = 0; q < kCountPer; q++) {
-    uint32_t j = base + q * kAgentBlock + threadIdx.x;
-    // 64-bit test: near the 2^32 - 256 agent limit the last block's slots wrap
-    act[q] = uint64_t(base) + q * kAgentBlock + threadIdx.x < total;
-    k[q] = 0;
+  for (int q = 0; q < kSortPer; q++) {
+    uint32_t j;
+    t.act[q] = sort_slot(g, base, q, j);
+    t.k[q] = t.r[q] = 0;
+  }
+#pragma unroll
+  for (int q = 0; q < kSortPer; q++) {
+    if (uint64_t(base) + q * kAgentBlock >= g.total) break;  // uniform; no block_inst entry
+    const uint32_t first = base + q * kAgentBlock;
+    const uint32_t last = min(first + kAgentBlock, g.total) - 1u;
+    const uint32_t j = first + threadIdx.x;
+    for (uint32_t ii = g.block_inst[first / kAgentBlock];; ii++) {  // block-uniform walk
+      const Instance in = g.insts[ii];
+      const uint32_t end = in.agent_off + in.agent_count;
+      if (t.act[q] && j >= in.agent_off && j < end)
+        t.k[q] = key_of(x[q], y[q], th[q], in, g.params[ii], g.cell_log2, g.sort_key);
+      if (last < end || ii + 1u >= g.ninst) break;
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < kSortPer; q++)
+    if (t.act[q]) s_tag[t.entry(q)] = t.k[q];
+  __syncthreads();
+  bool shared = false;
+#pragma unroll
+  for (int q = 0; q < kSortPer; q++)
+    if (t.act[q]) {
+      shared |= s_tag[t.entry(q)] != t.k[q];
+      t.r[q] = atomicAdd(&s_cnt[t.entry(q)], 1u);
+    }
+  t.local = !__syncthreads_or(shared);
+  return t;
+}
+
+// The fallback: add(bin, n) by one lane for n lanes of a wave in the bin, old its
+// result and `below` the rank among them.  The first few distinct bins of a wave are
+// taken together (agents that crowd a few distant bins), the others lane by lane
+// (agents in any order, as before the first re-sort, share almost none).
+constexpr int kWaveBins = 4;
+template <class Add, class Use>
+__device__ inline void each_wave_bin(const Keys& t, Add&& add, Use&& use) {
+  const int lane = static_cast<int>(threadIdx.x & 63u);
+#pragma unroll
+  for (int q = 0; q < kSortPer; q++) {
+    bool todo = t.act[q];
+    for (int n = 0; n < kWaveBins; n++) {
+      const uint64_t pending = __ballot(todo);
+      if (!pending) break;
+      const int leader = __builtin_ctzll(pending);
+      const bool mine = todo && t.k[q] == static_cast<uint32_t>(__shfl(t.k[q], leader));
+      const uint64_t same = __ballot(mine);
+      uint32_t old = 0;
+      if (lane == leader) old = add(t.k[q], static_cast<uint32_t>(__popcll(same)));
+      old = __shfl(old, leader);
+      if (mine) use(q, old, static_cast<uint32_t>(__popcll(same & ((uint64_t(1) << lane) - 1u))));
+      todo = todo && !mine;
+    }
+    if (todo) use(q, add(t.k[q], 1u), 0u);
+  }
+}
+
+// count[bin] += the bin's agents.  All of a thread's agents are loaded before any
+// is used: with one agent per thread the chain of load, barrier and atomic per
+// block set the kernel's time, not the bandwidth.
+__global__ __launch_bounds__(kAgentBlock) void count_kernel(SortArgs g, AgentSoA a, int pos64,
+                                                            uint32_t* count) {
+  __shared__ uint32_t s_cnt[kLocalBins], s_tag[kLocalBins];
+  const uint32_t base = sort_base(g);
+  float px[kSortPer], py[kSortPer], pth[kSortPer];
+  // the heading only enters refined keys: the plain key loads positions only
+  const bool heading = g.sort_key != 0u;
+#pragma unroll
+  for (int q = 0; q < kSortPer; q++) {
+    uint32_t j;
     px[q] = py[q] = pth[q] = 0.0f;
-    if (act[q]) {
+    if (sort_slot(g, base, q, j)) {
       px[q] = pos64 ? static_cast<float>(a.x64[j]) : a.x[j];
       py[q] = pos64 ? static_cast<float>(a.y64[j]) : a.y[j];
       if (heading) pth[q] = a.th[j];
     }
   }
-#pragma unroll
-  for (int q = 0; q < kCountPer; q++) {
-    if (uint64_t(base) + q * kAgentBlock >= total) break;  // block-uniform; no block_inst entry
-    uint32_t first = base + q * kAgentBlock;
-    uint32_t last = min(first + kAgentBlock, total) - 1u;
-    uint32_t j = first + threadIdx.x;
-    for (uint32_t ii = block_inst[first / kAgentBlock];; ii++) {  // block-uniform walk
-      const Instance in = insts[ii];
-      uint32_t end = in.agent_off + in.agent_count;
-      if (act[q] && j >= in.agent_off && j < end)
-        k[q] = key_of(px[q], py[q], pth[q], in, params[ii], cell_log2, sort_key);
-      if (last < end || ii + 1u >= ninst) break;
-    }
-  }
-  if (threadIdx.x == 0) {
-    s_min = 0xffffffffu;
-    s_max = 0u;
-  }
-  __syncthreads();
-  // wave min/max by butterfly, then one LDS atomic per wave (256 same-address
-  // LDS atomics per block serialised and dominated the kernel)
-  uint32_t wmin = 0xffffffffu, wmax = 0u;
-#pragma unroll
-  for (int q = 0; q < kCountPer; q++)
-    if (act[q]) {
-      wmin = min(wmin, k[q]);
-      wmax = max(wmax, k[q]);
-    }
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    wmin = min(wmin, static_cast<uint32_t>(__shfl_xor(static_cast<int>(wmin), off)));
-    wmax = max(wmax, static_cast<uint32_t>(__shfl_xor(static_cast<int>(wmax), off)));
-  }
-  if ((threadIdx.x & 63u) == 0u) {
-    atomicMin(&s_min, wmin);
-    atomicMax(&s_max, wmax);
-  }
-  __syncthreads();
-  const uint32_t kmin = s_min, kmax = s_max;
-  const bool local = kmax >= kmin && kmax - kmin < kLocalBins;  // block-uniform
-  if (local)
-    for (uint32_t i = threadIdx.x; i <= kmax - kmin; i += kAgentBlock) s_cnt[i] = 0u;
-  __syncthreads();
-
-  uint32_t r[kCountPer];
-#pragma unroll
-  for (int q = 0; q < kCountPer; q++) r[q] = 0;
-  if (local) {
-    // rank inside the block: one LDS atomic per agent (lanes of a bin take
-    // distinct old values; the few bins of a block spread over the banks)
-#pragma unroll
-    for (int q = 0; q < kCountPer; q++)
-      if (act[q]) r[q] = atomicAdd(&s_cnt[k[q] - kmin], 1u);
-  } else {
-    // wide key range: one global atomic per distinct bin of each wave
-    uint32_t lane = threadIdx.x & 63u;
-    uint64_t below = (uint64_t(1) << lane) - 1u;
-#pragma unroll
-    for (int q = 0; q < kCountPer; q++) {
-      uint64_t pending = __ballot(act[q]);
-      while (pending) {
-        int leader = __builtin_ctzll(pending);
-        uint32_t lk = __shfl(k[q], leader);
-        uint64_t same = __ballot(act[q] && k[q] == lk);
-        uint32_t b = 0;
-        if (static_cast<int>(lane) == leader) b = atomicAdd(count + lk, __popcll(same));
-        b = __shfl(b, leader);
-        if (act[q] && k[q] == lk) r[q] = b + __popcll(same & below);
-        pending &= ~same;
-      }
-    }
-  }
-  if (local) {
-    __syncthreads();
-    for (uint32_t i = threadIdx.x; i <= kmax - kmin; i += kAgentBlock) {
-      uint32_t c = s_cnt[i];
-      if (c) s_base[i] = atomicAdd(count + kmin + i, c);
-    }
-    __syncthreads();
-#pragma unroll
-    for (int q = 0; q < kCountPer; q++)
-      if (act[q]) r[q] += s_base[k[q] - kmin];
+  const Keys t = block_keys(g, base, px, py, pth, s_cnt, s_tag);
+  if (!t.local) {
+    each_wave_bin(
+        t, [&](uint32_t k, uint32_t n) { return atomicAdd(count + k, n); },
+        [](int, uint32_t, uint32_t) {});
+    return;
   }
 #pragma unroll
-  for (int q = 0; q < kCountPer; q++)
-    if (act[q]) {
-      uint32_t j = base + q * kAgentBlock + threadIdx.x;
-      rank[j] = r[q];
-    }
+  for (int q = 0; q < kSortPer; q++)  // by the first agent of each bin
+    if (t.act[q] && t.r[q] == 0u) atomicAdd(count + t.k[q], s_cnt[t.entry(q)]);
 }
 
 // Exclusive scan of one tile of `in` into `out` (in place allowed); writes
@@ -243,53 +252,123 @@ __global__ __launch_bounds__(kScanBlock) void scan_add_kernel(uint32_t* out, uin
     if (base + k < n) out[base + k] += add;
 }
 
-// Moves each agent to offset[bin] + rank.  The bin is recomputed from the
-// position the scatter reads anyway (the same float arithmetic as the count
-// kernel's, so the same bin) instead of being stored by the count kernel and
-// read back: 8 bytes per agent less traffic, ~15% of the re-sort.
-__global__ __launch_bounds__(kAgentBlock) void scatter_kernel(
-    AgentSoA src, AgentSoA dst, const Instance* insts, const DevParams* params,
-    const uint32_t* block_inst, uint32_t ninst, uint32_t n, int pos64, uint32_t cell_log2,
-    uint32_t sort_key, int xcd_remap, const uint32_t* rank, const uint32_t* offset) {
-  const uint32_t blk = xcd_remap ? xcd_logical_block(blockIdx.x, gridDim.x) : blockIdx.x;
-  uint32_t first = blk * kAgentBlock;
-  uint32_t last = min(first + kAgentBlock, n) - 1u;
-  uint32_t j = first + threadIdx.x;
-  bool act = j < n;
-  double x64 = 0.0, y64 = 0.0;
-  float x = 0.0f, y = 0.0f, th = 0.0f;
-  if (act) {
-    th = src.th[j];
-    if (pos64) {
-      x64 = src.x64[j];
-      y64 = src.y64[j];
-      x = static_cast<float>(x64);
-      y = static_cast<float>(y64);
-    } else {
-      x = src.x[j];
-      y = src.y[j];
-    }
-  }
-  uint32_t k = 0;
-  for (uint32_t ii = block_inst[blk];; ii++) {  // block-uniform walk
-    const Instance in = insts[ii];
-    uint32_t end = in.agent_off + in.agent_count;
-    if (act && j >= in.agent_off && j < end) k = key_of(x, y, th, in, params[ii], cell_log2, sort_key);
-    if (last < end || ii + 1u >= ninst) break;
-  }
-  if (!act) return;
-  const uint32_t d = offset[k] + rank[j];
-  if (d >= n) return;  // unreachable: count and scatter compute the same keys
-  if (pos64) {
-    dst.x64[d] = x64;
-    dst.y64[d] = y64;
+// Moves each agent into its bin's range of slots, [offset[bin], offset[bin] +
+// count[bin]), from the end of the range down: count[bin] is the part of it that is
+// still free.  Bins are recomputed from the positions, by the count kernel's
+// arithmetic.
+//
+// The vector L1 takes a divergent store one lane a cycle, so writing each agent
+// where it goes costs 64 accesses per array and wave (count and scatter of 2^24
+// agents, f32: 117 + 230 us).  The workgroup orders its agents by bin in LDS
+// instead (each bin's agents are reserved one run of slots) and writes the runs:
+// 52 + 190 us; 8192^2 bf16 with f64 positions and 2^26 agents 443 + 930 -> 288 + 777;
+// 64 instances of 256^2 to 2048^2 with 5 * 10^7 agents 516 + 716 -> 160 + 670.
+// Bound by the LDS passes and the reservation's round trip.
+template <bool P64>
+__global__ __launch_bounds__(kAgentBlock) void scatter_kernel(SortArgs g, AgentSoA src,
+                                                              AgentSoA dst, uint32_t* count,
+                                                              const uint32_t* offset) {
+
+  __shared__ uint32_t s_cnt[kLocalBins];   // agents per bin, then the bin's first position
+  __shared__ uint32_t s_base[kLocalBins];  // the bin's first slot
+  // s_dst: the waves' sums, then each position's slot
+  __shared__ uint32_t s_dst[kSortSlots], s_th[kSortSlots], s_v[kSortSlots], s_id[kSortSlots];
+  using pos = std::conditional_t<P64, double, float>;
+  __shared__ pos s_x[kSortSlots], s_y[kSortSlots];
+  const pos *sx, *sy;
+  pos *dx, *dy;
+  if constexpr (P64) {
+    sx = src.x64, sy = src.y64, dx = dst.x64, dy = dst.y64;
   } else {
-    dst.x[d] = x;
-    dst.y[d] = y;
+    sx = src.x, sy = src.y, dx = dst.x, dy = dst.y;
   }
-  dst.th[d] = th;
-  dst.v[d] = src.v[j];
-  dst.id[d] = src.id[j];
+  const uint32_t base = sort_base(g);
+  pos x[kSortPer], y[kSortPer];
+  float fx[kSortPer], fy[kSortPer], th[kSortPer], v[kSortPer];
+  uint32_t id[kSortPer];
+#pragma unroll
+  for (int q = 0; q < kSortPer; q++) {
+    uint32_t j;
+    x[q] = y[q] = 0;
+    th[q] = v[q] = 0.0f;
+    id[q] = 0;
+    if (sort_slot(g, base, q, j)) {
+      x[q] = sx[j];
+      y[q] = sy[j];
+      th[q] = src.th[j];
+      v[q] = src.v[j];
+      id[q] = src.id[j];
+    }
+    fx[q] = static_cast<float>(x[q]);
+    fy[q] = static_cast<float>(y[q]);
+  }
+  const Keys t = block_keys(g, base, fx, fy, th, s_cnt, s_base);
+  // the first of n slots for agents of bin k
+  auto reserve = [&](uint32_t k, uint32_t n) { return offset[k] + atomicSub(count + k, n) - n; };
+  if (!t.local) {
+    each_wave_bin(t, reserve, [&](int q, uint32_t first, uint32_t rank) {
+      const uint32_t d = first + rank;
+      if (d >= g.total) return;  // unreachable: the count kernel's bins
+      dx[d] = x[q];
+      dy[d] = y[q];
+      dst.th[d] = th[q];
+      dst.v[d] = v[q];
+      dst.id[d] = id[q];
+    });
+    return;
+  }
+#pragma unroll
+  for (int q = 0; q < kSortPer; q++)  // by the first agent of each bin
+    if (t.act[q] && t.r[q] == 0u) s_base[t.entry(q)] = reserve(t.k[q], s_cnt[t.entry(q)]);
+  // each bin's first position: thread i scans kPer consecutive bins
+  constexpr uint32_t kPer = kLocalBins / kAgentBlock;
+  const uint32_t lane = threadIdx.x & 63u;
+  uint32_t c[kPer], sum = 0;
+#pragma unroll
+  for (uint32_t i = 0; i < kPer; i++) {
+    c[i] = s_cnt[threadIdx.x * kPer + i];
+    sum += c[i];
+  }
+  uint32_t run = sum;  // inclusive, over the wave
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const uint32_t n = __shfl_up(run, off);
+    if (lane >= static_cast<uint32_t>(off)) run += n;
+  }
+  if (lane == 63u) s_dst[threadIdx.x >> 6] = run;
+  __syncthreads();
+  run -= sum;
+  for (uint32_t i = 0; i < threadIdx.x >> 6; i++) run += s_dst[i];
+#pragma unroll
+  for (uint32_t i = 0; i < kPer; i++) {
+    s_cnt[threadIdx.x * kPer + i] = run;
+    run += c[i];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < kSortPer; q++)
+    if (t.act[q]) {
+      const uint32_t p = s_cnt[t.entry(q)] + t.r[q];
+      s_dst[p] = s_base[t.entry(q)] + t.r[q];
+      s_x[p] = x[q];
+      s_y[p] = y[q];
+      s_th[p] = __float_as_uint(th[q]);
+      s_v[p] = __float_as_uint(v[q]);
+      s_id[p] = id[q];
+    }
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < kSortPer; q++) {
+    const uint32_t p = q * kAgentBlock + threadIdx.x;
+    if (!t.act[q]) continue;  // the workgroup's n agents hold positions 0 .. n - 1
+    const uint32_t d = s_dst[p];
+    if (d >= g.total) continue;  // unreachable: the count kernel's bins
+    dx[d] = s_x[p];
+    dy[d] = s_y[p];
+    dst.th[d] = __uint_as_float(s_th[p]);
+    dst.v[d] = __uint_as_float(s_v[p]);
+    dst.id[d] = s_id[p];
+  }
 }
 
 __global__ __launch_bounds__(kAgentBlock) void canonical_copy_kernel(
@@ -426,13 +505,15 @@ void launch_morton_sort(const Pool& pool, const AgentSoA& src, const AgentSoA& d
                         const SortScratch& s, hipStream_t stream) {
   if (pool.total_agents == 0) return;
   zero_u32_kernel<<<blocks_for(pool.total_bins, 256), 256, 0, stream>>>(s.count, pool.total_bins);
-  count_kernel<<<blocks_for(pool.total_agents, kCountSlots), kAgentBlock, 0, stream>>>(
-      src, pool.inst, pool.params, pool.agent_block_inst, pool.count, pool.total_agents,
-      pool.pos64, pool.sort_cell_log2, pool.sort_key, pool.xcd_remap, s.rank, s.count);
+  const SortArgs g{pool.inst,          pool.params,   pool.agent_block_inst, pool.count,
+                   pool.total_agents,  pool.sort_cell_log2, pool.sort_key,   pool.xcd_remap};
+  const uint32_t nb = blocks_for(pool.total_agents, kSortSlots);
+  count_kernel<<<nb, kAgentBlock, 0, stream>>>(g, src, pool.pos64, s.count);
   scan(s, s.count, pool.total_bins, s.offset, 0, stream);
-  scatter_kernel<<<blocks_for(pool.total_agents, kAgentBlock), kAgentBlock, 0, stream>>>(
-      src, dst, pool.inst, pool.params, pool.agent_block_inst, pool.count, pool.total_agents,
-      pool.pos64, pool.sort_cell_log2, pool.sort_key, pool.xcd_remap, s.rank, s.offset);
+  if (pool.pos64)
+    scatter_kernel<true><<<nb, kAgentBlock, 0, stream>>>(g, src, dst, s.count, s.offset);
+  else
+    scatter_kernel<false><<<nb, kAgentBlock, 0, stream>>>(g, src, dst, s.count, s.offset);
   if (pool.items) {  // work list of the tiled agent pass
     uint32_t nt = pool.total_tiles;
     tile_count_kernel<<<blocks_for(nt, 256), 256, 0, stream>>>(
