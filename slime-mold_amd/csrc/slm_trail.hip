@@ -989,7 +989,14 @@ void launch_gauss_t(const Pool& pool, const void* in, void* out, hipStream_t str
 
 void plan_trail(Instance& in, int storage, uint32_t fixed_rows) {
   uint32_t v = storage == SLM_STORAGE_F32 ? 4u : 8u;
-  if (in.width >= v) {
+  // Strips, except where rows are no whole number of them and there are too few to
+  // fill the chip (one cell per lane then makes more waves): strips / cells take, us,
+  // 407 x 876 f16 (219 strip units) 7.5 / 6.3, 1001 x 701 f16 (352) 8.0 / 7.8,
+  // 1365 x 767 bf16 (576) 7.9 / 9.1.  A tile height that was asked for means strips.
+  constexpr uint32_t kFewStrips = 400;
+  const uint64_t strips = static_cast<uint64_t>((in.width + 64u * v - 1u) / (64u * v)) *
+                          ((in.height + 3u) / 4u);
+  if (in.width >= v && (in.width % v == 0 || fixed_rows || strips >= kFewStrips)) {
     in.ntx = (in.width + 64u * v - 1u) / (64u * v);
     // Rows per strip unit: fixed, or 4.  The shortest tiles are loaded whole, keep the
     // most waves, and their halo rows are found in the L2: at every size they take
