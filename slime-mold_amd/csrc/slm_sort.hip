@@ -154,8 +154,8 @@ __device__ inline Keys block_keys(const SortArgs& g, uint32_t base, const float 
   return t;
 }
 
-// The fallback: add(bin, n) by one lane for n lanes of a wave in the bin, old its
-// result and `below` the rank among them.  The first few distinct bins of a wave are
+// The fallback: old = add(bin, n) by one lane for n lanes of a wave in the bin, then
+// use(q, old, rank among them) by each.  The first few distinct bins of a wave are
 // taken together (agents that crowd a few distant bins), the others lane by lane
 // (agents in any order, as before the first re-sort, share almost none).
 constexpr int kWaveBins = 4;
