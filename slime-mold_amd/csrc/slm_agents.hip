@@ -814,14 +814,16 @@ __device__ inline float wrap_up(float r, float b) {
 }
 // `turn` for |angle| < kQuickAngle and turn_speed <= kQuickTurn: the distance to
 // either target is then 2 pi to within 2.5e-4, above turn_speed, so the turn is
-// -turn_speed or +turn_speed, the sign of rv - lv (exact: f32 subtraction keeps
-// denormals, so it is 0 only for equal values).
+// -turn_speed or +turn_speed, the sign of rv - lv.  That is 0 only for equal values
+// (f32 subtraction keeps denormals) and NaN only for values that compare neither way
+// (two infinities, as f16 cells beyond 65504 are, or a NaN sample): |rv - lv| > 0 is
+// lv < rv or lv > rv.
 __device__ inline float turn_quick(float angle, float lv, float rv, float cv, float turn_speed,
                                    uint32_t sign) {
   const float d = rv - lv;
   const float turned =
       angle + __uint_as_float(__float_as_uint(turn_speed) ^ (__float_as_uint(d) & sign));
-  const bool straight = (d == 0.0f) | ((cv > lv) & (cv > rv));
+  const bool straight = !(__builtin_fabsf(d) > 0.0f) | ((cv > lv) & (cv > rv));
   return straight ? angle : turned;
 }
 
