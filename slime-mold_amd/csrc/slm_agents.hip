@@ -1030,8 +1030,6 @@ __device__ inline void tile_update(const AgentSoA& a, uint32_t j, uint32_t slot,
   __builtin_amdgcn_s_setprio(0);
 }
 
-template <bool P64>
-constexpr int kTileBlockOf = P64 ? 512 : 1024;
 constexpr uint32_t kMinStagedAgents = 256;  // sparser items read global memory
 
 __device__ inline uint32_t compact_bits(uint32_t v) {  // even bits -> 16 bits
@@ -1089,12 +1087,12 @@ __device__ inline TileWindow tile_window(const WorkItem& wi, const Instance& in,
 }
 
 template <int S, bool P64, bool kOne>
-__global__ __launch_bounds__(kTileBlockOf<P64>)
+__global__ __launch_bounds__(tile_block(P64))
     __attribute__((amdgpu_waves_per_eu(P64 ? 4 : 8))) void agents_tiled_kernel(
         TiledArgs args, const Instance* __restrict__ insts, const DevParams* __restrict__ params) {
   using elem = typename TrailRead<S>::elem;
   constexpr int V = static_cast<int>(16 / sizeof(elem));  // cells per 16-byte chunk
-  constexpr int kTileBlock = kTileBlockOf<P64>;
+  constexpr int kTileBlock = tile_block(P64);
   constexpr int kDeep = (static_cast<int>(kTileLds) / (V * 4) + kTileBlock - 1) / kTileBlock;  // chunks per lane
   extern __shared__ __align__(16) char smem[];
   const uint32_t t = threadIdx.x;
@@ -1350,7 +1348,7 @@ void prime_persistent_agents() {
 void launch_agents_tiled(const Pool& pool, const AgentSoA& a, void* trail, uint32_t drift_steps,
                          hipStream_t stream) {
   if (pool.total_agents == 0 || pool.max_items == 0) return;
-  const int block = pool.pos64 ? kTileBlockOf<true> : kTileBlockOf<false>;
+  const int block = tile_block(pool.pos64 != 0);
   TiledArgs args{a, trail, pool.items, drift_steps};
   auto go = [&](auto* one, auto* many) {
     if (pool.count == 1)

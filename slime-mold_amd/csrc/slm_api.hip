@@ -1482,7 +1482,13 @@ class Engine {
       // offset[total_bins] closes the last bin: the scan fills the rest
       SLM_HIP(hipMemcpy(sort_.offset + total_bins_, &total_agents_, 4, hipMemcpyHostToDevice));
       total_tiles_ = static_cast<uint32_t>(tiles);
-      max_items_ = total_tiles_ + blocks_for(total_agents_, kItemAgents);
+      // A tile of n agents has max(1, n / kItemAgents to the nearest) items, and only
+      // tiles that reach into the grid have agents: the list is bounded by these, not by
+      // total_tiles_, which counts the whole Morton square (2^22 tiles for 2048 of them
+      // on a 131072 x 64 grid, more workgroups than a launch can have).
+      uint64_t items = blocks_for(total_agents_, kItemAgents);
+      for (const Instance& in : inst) items += std::min<uint64_t>(grid_tiles(in), in.agent_count);
+      max_items_ = static_cast<uint32_t>(items);
       std::vector<uint32_t> tmap(total_tiles_);
       for (size_t k = 0; k < spec.size(); k++)
         for (uint32_t t = 0; t < inst[k].tiles; t++) tmap[inst[k].tile_off + t] = static_cast<uint32_t>(k);
@@ -1514,6 +1520,11 @@ class Engine {
 
   bool sort_due(uint64_t step_index) const {
     return sorting() && step_index % cfg.resort_interval == 0;
+  }
+
+  // Whether a workgroup for every work item fits one launch (2^32 threads).
+  bool tiles_launchable() const {
+    return static_cast<uint64_t>(max_items_) * tile_block(pos64()) < (1ull << 32);
   }
 
   // Whether the pool's agents sense through tile windows of the library's own
@@ -1574,7 +1585,7 @@ class Engine {
   // the same bits.
   void enqueue_agents(const Pool& p, uint64_t step) {
     const uint32_t drift = sorting() ? static_cast<uint32_t>(step % cfg.resort_interval) + 1u : 0u;
-    if (sorting() && tiles_ready_ &&
+    if (sorting() && tiles_ready_ && tiles_launchable() &&
         ((cfg.flags & SLM_FLAG_TILED_SENSING) || drift <= tile_steps_))
       launch_agents_tiled(p, agents_[acur_], trail_[cur_], drift, stream);
     else

@@ -130,6 +130,8 @@ constexpr uint32_t gauss_th(int storage, int rclass) {
 }
 
 constexpr uint32_t kTileLog2 = 6;  // sensing tiles of 64 x 64 cells
+// Threads of a tile's workgroup (f64 positions need more registers).
+constexpr int tile_block(bool pos64) { return pos64 ? 512 : 1024; }
 constexpr uint32_t kTileLds = 81920;  // LDS bytes of a tile's window: two workgroups to a CU
 
 // The margin that a tile's window has around it, `steps` steps after the re-sort:
@@ -286,6 +288,11 @@ uint64_t plan_bins(Instance& in, uint32_t cell_log2);
 // Tiles of 2^tile_log2 cells (>= the bin edge) for tiled sensing: fills
 // tile_log2 and tiles.
 void plan_tiles(Instance& in, uint32_t cell_log2, uint32_t tile_log2);
+// The tiles that reach into the grid.
+inline uint64_t grid_tiles(const Instance& in) {
+  const uint64_t side = uint64_t(1) << in.tile_log2;
+  return ((in.width + side - 1) >> in.tile_log2) * ((in.height + side - 1) >> in.tile_log2);
+}
 
 // ---- launchers (all asynchronous on `stream`) ----------------------------
 void launch_agents(const Pool& pool, const AgentSoA& a, void* trail, hipStream_t stream);
