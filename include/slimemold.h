@@ -117,8 +117,9 @@ typedef struct slm_config {
  * sensor reach plus drift since the re-sort) in LDS and sense from there; agents
  * that the window does not cover, and tiles whose window does not fit 80 KiB, read
  * global memory, so results are unchanged.  Without the flag the library does so
- * by itself where it pays (from 2^21 agents on, one agent to four cells, windows
- * that fit); with it, wherever there is a re-sort. */
+ * by itself where it pays (from 2^21 agents on, 2^22 with f64 positions, some 1600
+ * to a tile, windows that fit for a number of steps); with it, wherever there is a
+ * re-sort. */
 #define SLM_FLAG_TILED_SENSING 0x4u
 /* With BF16 storage: the trail pass stores each cell rounded up with
  * probability equal to the discarded fraction of its f32 value, instead of to
@@ -366,6 +367,11 @@ typedef struct slm_tuning {
 #define SLM_SORT_AT_SENSOR 0x10u
 
 int slm_get_tuning(const slm_sim* sim, slm_tuning* out);
+/* How the agents of the next step will sense: 0 = from global memory, 1 = through
+ * tile windows (SLM_FLAG_TILED_SENSING, or the library's choice), 2 = through
+ * workgroup windows.  The choice changes from step to step: tile windows need a
+ * re-sort before and fit for a number of steps after it. */
+int slm_get_sensing(const slm_sim* sim, uint32_t* out);
 /* Applies a tuning.  Agent and trail state, the step count and the parameters
  * are kept; captured graphs are rebuilt on the next slm_step. */
 int slm_set_tuning(slm_sim* sim, const slm_tuning* tuning);
@@ -388,6 +394,7 @@ int slm_set_tuning(slm_sim* sim, const slm_tuning* tuning);
 int slm_autotune(slm_sim* sim, uint32_t trial_steps, slm_tuning* out);
 
 int slm_batch_get_tuning(const slm_batch* batch, slm_tuning* out);
+int slm_batch_get_sensing(const slm_batch* batch, uint32_t* out);
 int slm_batch_set_tuning(slm_batch* batch, const slm_tuning* tuning);
 int slm_batch_autotune(slm_batch* batch, uint32_t trial_steps, slm_tuning* out);
 

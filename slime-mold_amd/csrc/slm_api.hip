@@ -355,8 +355,8 @@ class Engine {
     p.total_tiles = total_tiles_;
     p.tile_inst = tile_inst_d_;
     // the re-sort builds the tiled pass's work list only when that pass is on
-    // (turning it on re-lays the tables and waits for the next re-sort)
-    p.items = (cfg.flags & SLM_FLAG_TILED_SENSING) || auto_tiles() ? items_d_ : nullptr;
+    // (turned on later, it waits for the next re-sort)
+    p.items = uses_tiles() ? items_d_ : nullptr;
     p.max_items = max_items_;
     p.agents_per_group = cfg.agents_per_group;
     p.preload_rows = preload_rows_;
@@ -735,6 +735,11 @@ class Engine {
   }
 
   // ---- launch tuning ----------------------------------------------------------
+  uint32_t sensing() const {
+    if (senses_tiles(steps_done, sorts_at(steps_done) ? uses_tiles() : tiles_ready_)) return 1u;
+    return (cfg.flags & SLM_FLAG_WINDOW_SENSING) ? 2u : 0u;
+  }
+
   slm_tuning tuning() const {
     slm_tuning t;
     std::memset(&t, 0, sizeof t);
@@ -1157,11 +1162,12 @@ class Engine {
   int gauss_rclass_ = kGaussMaxR;  // Gaussian-pass LDS radius class (gauss_class)
   uint32_t preload_rows_ = 0;
   uint64_t total_cells_ = 0;
+  double window_tiles_ = 1;  // 64 x 64-cell tiles that reach into the instances' grids
   std::vector<uint32_t> window_steps_;  // per instance, for the current layout and parameters
   uint32_t tile_steps_ = 0;             // tile_steps_now for them
   uint32_t* tile_inst_d_ = nullptr;
   WorkItem* items_d_ = nullptr;
-  bool tiles_ready_ = false;  // the latest re-sort's work list matches the layout
+  bool tiles_ready_ = false;  // the latest re-sort built a work list, and it matches the layout
   uint64_t trail_elems_ = 0;
   // Captured chunks.  A chunk's launches depend on the current trail and
   // agent buffers and on where the chunk starts in the re-sort schedule
@@ -1446,6 +1452,8 @@ class Engine {
     }
     total_bins_ = sorting() ? static_cast<uint32_t>(bins) : 0;
     total_cells_ = total_cells;
+    window_tiles_ = 0;
+    for (const Instance& in : inst) window_tiles_ += grid_tiles(in.width, in.height, kTileLog2);
     SLM_HIP(hipMemcpy(inst_d_, inst.data(), inst.size() * sizeof(Instance), hipMemcpyHostToDevice));
     SLM_TRY(build_groups());
     window_steps_.assign(spec.size(), 0u);
@@ -1487,7 +1495,7 @@ class Engine {
       // total_tiles_, which counts the whole Morton square (2^22 tiles for 2048 of them
       // on a 131072 x 64 grid, more workgroups than a launch can have).
       uint64_t items = blocks_for(total_agents_, kItemAgents);
-      for (const Instance& in : inst) items += std::min<uint64_t>(grid_tiles(in), in.agent_count);
+      for (const Instance& in : inst) items += std::min(grid_tiles(in.width, in.height, in.tile_log2), uint64_t(in.agent_count));
       max_items_ = static_cast<uint32_t>(items);
       std::vector<uint32_t> tmap(total_tiles_);
       for (size_t k = 0; k < spec.size(); k++)
@@ -1527,20 +1535,32 @@ class Engine {
     return static_cast<uint64_t>(max_items_) * tile_block(pos64()) < (1ull << 32);
   }
 
+  // Whether any step senses through tile windows.
+  bool uses_tiles() const { return (cfg.flags & SLM_FLAG_TILED_SENSING) || tile_steps_ > 0u; }
+
   // Whether the pool's agents sense through tile windows of the library's own
   // accord: with the plain re-sort key, one launch per pass over the pool and no
-  // other sensing asked for, from 2^21 agents on and one agent to four cells.
-  // Measured (us per agent pass, global against tiled, re-sort every 20 steps):
-  // 2048^2 with 2^21 agents 38.8 against 31.6, with 2^20 25.0 either way, with
-  // 2^19 19.8 against 21.3; 4096^2 with 2^24 293 against 221, with 2^23 128
-  // against 109, with 2^22 (a quarter per cell) 77.7 against 78.2 and 69.4
-  // against 66.0; 256^2 with 2^18 17.4 against 20.4: fewer agents do not fill
-  // the chip with 1024-thread workgroups, sparser ones stage cells that few read.
+  // other sensing asked for, from 2^21 agents on (2^22 with f64 positions, whose
+  // workgroups hold half the waves) and with enough of them to a tile.  Fewer agents
+  // do not fill the chip with workgroups of whole tiles; tiles that hold few, or that
+  // the grid's edge cuts to slivers (the mean is weighed by the share of the tiles'
+  // area that is grid), stage cells that few read.  Agent pass against the global
+  // one's time, by agents per tile times that share:
+  //    < 1000   64 instances of 257^2, 2^21 agents 1.02, 839 of 200^2 1.09, 8192 of 16^2 2.7
+  //     1526    210 of 100^2 1.19, 419 of 200^2 1.05, with f64 positions 1.1 to 1.4
+  //     1582    93 of 300^2, 2^22 agents 0.83 (bf16 0.94, f64 0.96 to 1.00)
+  //     1975    82 of 160^2, 2^21 agents 1.03, 2^22 0.92 (f64 1.05 to 1.13, 0.96 to 1.04)
+  //     2048    one 2048^2 0.86, 1024 of 64^2 0.91 (f64 0.85, 1.0)
+  //     4096    one 2048^2 0.75, one 4096^2 0.68, 512 of 64^2 0.83
   bool auto_tiles() const {
-    constexpr uint32_t kMinAgents = 1u << 21;
+    const uint64_t min_agents = pos64() ? 1u << 22 : 1u << 21;
+    const double min_per_tile = pos64() ? 1900.0 : 1550.0;
+    constexpr double kTileCells = double(1u << (2 * kTileLog2));
+    const double per_tile = static_cast<double>(total_agents_) / window_tiles_ *
+                            (static_cast<double>(total_cells_) / (window_tiles_ * kTileCells));
     return sorting() && groups_.size() <= 1 && cfg.sort_key == 0u &&
            !(cfg.flags & (SLM_FLAG_WINDOW_SENSING | SLM_FLAG_PERSISTENT)) &&
-           total_agents_ >= kMinAgents && total_agents_ >= total_cells_ / 4u;
+           total_agents_ >= min_agents && per_tile >= min_per_tile;
   }
 
   // The most steps after a re-sort, up to the interval, at which instance k's tile
@@ -1565,9 +1585,15 @@ class Engine {
   }
 
   // The most steps after a re-sort at which at least half of the agents sense
-  // through windows; 0 where the pool does not.
+  // through windows; 0 where the pool does not.  Building the work list is six more
+  // launches of about 3 us at each re-sort, and windows save about 2 us a step for
+  // each 2^20 agents: they are taken where the steps they serve win that back.
   uint32_t tile_steps_now() const {
-    if (!auto_tiles()) return 0;
+    constexpr uint64_t kMinAgentSteps = 10u << 20;
+    const uint32_t steps = auto_tiles() ? half_window_steps() : 0u;
+    return static_cast<uint64_t>(steps) * total_agents_ >= kMinAgentSteps ? steps : 0u;
+  }
+  uint32_t half_window_steps() const {
     std::vector<std::pair<uint32_t, uint64_t>> by_steps;
     for (size_t k = 0; k < spec.size(); k++) by_steps.push_back({window_steps_[k], spec[k].agents});
     std::sort(by_steps.begin(), by_steps.end());
@@ -1580,14 +1606,22 @@ class Engine {
     return 0;
   }
 
+  // Absolute step `step`'s steps since its re-sort, itself included (0: never re-sorted).
+  uint32_t drift_at(uint64_t step) const {
+    return sorting() ? static_cast<uint32_t>(step % cfg.resort_interval) + 1u : 0u;
+  }
+  // Whether that step senses through tile windows, with (ready) a work list or without.
+  bool senses_tiles(uint64_t step, bool ready) const {
+    return sorting() && ready && tiles_launchable() &&
+           ((cfg.flags & SLM_FLAG_TILED_SENSING) || drift_at(step) <= tile_steps_);
+  }
+
   // Tiled sensing (when asked for, or where it pays: auto_tiles) once a re-sort
   // has laid agents out by tile; otherwise the global-memory pass.  Both give
   // the same bits.
   void enqueue_agents(const Pool& p, uint64_t step) {
-    const uint32_t drift = sorting() ? static_cast<uint32_t>(step % cfg.resort_interval) + 1u : 0u;
-    if (sorting() && tiles_ready_ && tiles_launchable() &&
-        ((cfg.flags & SLM_FLAG_TILED_SENSING) || drift <= tile_steps_))
-      launch_agents_tiled(p, agents_[acur_], trail_[cur_], drift, stream);
+    if (senses_tiles(step, tiles_ready_))
+      launch_agents_tiled(p, agents_[acur_], trail_[cur_], drift_at(step), stream);
     else
       launch_agents(p, agents_[acur_], trail_[cur_], stream);
   }
@@ -1595,7 +1629,7 @@ class Engine {
   void enqueue_sort(const Pool& p) {
     launch_morton_sort(p, agents_[acur_], agents_[acur_ ^ 1], sort_, stream);
     acur_ ^= 1;
-    tiles_ready_ = true;
+    tiles_ready_ = p.items != nullptr;
   }
 
   // Absolute step `step`; `between` runs after the agent pass is enqueued and
@@ -2051,7 +2085,7 @@ class Engine {
     for (uint32_t j = 0; j < chunk; j++) {  // the buffer swaps the captured steps make
       if (tc.sorted[j]) {
         acur_ ^= 1;
-        tiles_ready_ = true;
+        tiles_ready_ = uses_tiles();
       }
       cur_ ^= 1;
     }
@@ -2363,6 +2397,14 @@ int slm_get_tuning(const slm_sim* s, slm_tuning* out) {
   SLM_ENTRY_BEGIN
   if (!s || !s->eng || !out) return fail(SLM_ERR_INVALID_ARGUMENT, "NULL argument");
   *out = s->eng->tuning();
+  return SLM_OK;
+  SLM_ENTRY_END
+}
+
+int slm_get_sensing(const slm_sim* s, uint32_t* out) {
+  SLM_ENTRY_BEGIN
+  if (!s || !s->eng || !out) return fail(SLM_ERR_INVALID_ARGUMENT, "NULL argument");
+  *out = s->eng->sensing();
   return SLM_OK;
   SLM_ENTRY_END
 }
@@ -2733,6 +2775,14 @@ int slm_batch_get_tuning(const slm_batch* b, slm_tuning* out) {
   SLM_ENTRY_BEGIN
   if (!b || !b->eng || !out) return fail(SLM_ERR_INVALID_ARGUMENT, "NULL argument");
   *out = b->eng->tuning();
+  return SLM_OK;
+  SLM_ENTRY_END
+}
+
+int slm_batch_get_sensing(const slm_batch* b, uint32_t* out) {
+  SLM_ENTRY_BEGIN
+  if (!b || !b->eng || !out) return fail(SLM_ERR_INVALID_ARGUMENT, "NULL argument");
+  *out = b->eng->sensing();
   return SLM_OK;
   SLM_ENTRY_END
 }

@@ -288,10 +288,10 @@ uint64_t plan_bins(Instance& in, uint32_t cell_log2);
 // Tiles of 2^tile_log2 cells (>= the bin edge) for tiled sensing: fills
 // tile_log2 and tiles.
 void plan_tiles(Instance& in, uint32_t cell_log2, uint32_t tile_log2);
-// The tiles that reach into the grid.
-inline uint64_t grid_tiles(const Instance& in) {
-  const uint64_t side = uint64_t(1) << in.tile_log2;
-  return ((in.width + side - 1) >> in.tile_log2) * ((in.height + side - 1) >> in.tile_log2);
+// The tiles of 2^tile_log2 cells that reach into a grid.
+inline uint64_t grid_tiles(uint64_t width, uint64_t height, uint32_t tile_log2) {
+  const uint64_t edge = (uint64_t(1) << tile_log2) - 1u;
+  return ((width + edge) >> tile_log2) * ((height + edge) >> tile_log2);
 }
 
 // ---- launchers (all asynchronous on `stream`) ----------------------------

@@ -219,9 +219,11 @@ SIGNATURES = {
     "slm_create_from_snapshot": [ctypes.c_void_p, ctypes.c_uint64, ctypes.c_int32,
                                  ctypes.POINTER(_P)],
     "slm_get_tuning": [_P, ctypes.POINTER(Tuning)],
+    "slm_get_sensing": [_P, ctypes.POINTER(ctypes.c_uint32)],
     "slm_set_tuning": [_P, ctypes.POINTER(Tuning)],
     "slm_autotune": [_P, ctypes.c_uint32, ctypes.POINTER(Tuning)],
     "slm_batch_get_tuning": [_P, ctypes.POINTER(Tuning)],
+    "slm_batch_get_sensing": [_P, ctypes.POINTER(ctypes.c_uint32)],
     "slm_batch_set_tuning": [_P, ctypes.POINTER(Tuning)],
     "slm_batch_autotune": [_P, ctypes.c_uint32, ctypes.POINTER(Tuning)],
 }

@@ -116,6 +116,13 @@ class Batch:
         N.check(N.lib().slm_batch_get_tuning(self.handle, ctypes.byref(t)))
         return t
 
+    def sensing(self) -> int:
+        """How the next step's agents sense: 0 global memory, 1 tile windows, 2 workgroup
+        windows."""
+        v = ctypes.c_uint32(0)
+        N.check(N.lib().slm_batch_get_sensing(self.handle, ctypes.byref(v)))
+        return v.value
+
     def set_tuning(self, tuning: "N.Tuning" = None, **fields) -> None:
         """Apply a tuning; keyword fields override those of `tuning` (or of
         the current one)."""

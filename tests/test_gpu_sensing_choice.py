@@ -1,0 +1,52 @@
+"""Which agent pass the library takes by itself, and that its results are the same."""
+import pytest
+
+from parity_util import assert_bitwise, preset
+
+pytestmark = pytest.mark.gpu
+
+# count x (width, height, agents): whole tiles with many agents sense through windows;
+# small instances, slivers and few agents to a tile do not
+POOLS = [
+    ([(1600, 900, 1 << 21)], "f32", False, 1),
+    ([(2048, 2048, 1 << 22)], "bf16", True, 1),
+    ([(2048, 2048, 1 << 21)], "f32", True, 0),
+    ([(1024, 1024, 1 << 20)], "f32", False, 0),
+    ([(2900, 2900, 1 << 21)], "f32", False, 0),
+    ([(512, 512, 1 << 18)] * 9, "f16", False, 1),
+    ([(64, 64, 4096)] * 520 + [(200, 3, 50)], "f32", False, 1),
+    ([(96, 96, 9216)] * 230, "f32", False, 0),
+    ([(16, 16, 256)] * 8200, "f32", False, 0),
+]
+
+
+@pytest.mark.parametrize("dims,storage,f64,want", POOLS,
+                         ids=lambda v: f"{len(v)}x{v[0][0]}x{v[0][1]}" if isinstance(v, list) else str(v))
+def test_choice_by_agents_per_tile(slm, dims, storage, f64, want):
+    specs = [slm.InstanceSpec(w, h, n, seed=k, params=preset(slm, "Default"))
+             for k, (w, h, n) in enumerate(dims)]
+    some = sorted({0, len(specs) // 2, len(specs) - 1})
+    out = []
+    for resort in (0, 10):
+        with slm.Batch(specs, storage=storage, resort_interval=resort, graph_chunk=0,
+                       f64_positions=f64) as b:
+            print(f"[sensing] {len(specs)} x {dims[0]} resort={resort}", flush=True)
+            assert b.sensing() == (want if resort else 0)
+            b.step(3)
+            assert b.sensing() == (want if resort else 0)
+            out.append([(b.read_agents(k), b.read_trail(k)) for k in some])
+    for k, (a0, t0), (a1, t1) in zip(some, *out):
+        assert_bitwise(a1, a0, f"agents {k}")
+        assert_bitwise(t1, t0, f"trail {k}")
+
+
+def test_choice_follows_the_steps_that_windows_serve(slm):
+    """Every second step re-sorted: the work list costs more than two steps win back."""
+    with slm.Simulation(1600, 900, 1 << 21, seed=1, params=preset(slm, "Default"),
+                        resort_interval=2) as sim:
+        assert sim.sensing() == 0
+        for interval in (5, 8):
+            sim.set_tuning(resort_interval=interval)
+            assert sim.sensing() == 1
+        sim.set_params(preset(slm, "Snake"))  # sensors that no window covers
+        assert sim.sensing() == 0
