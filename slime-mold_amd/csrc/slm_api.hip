@@ -1170,13 +1170,15 @@ class Engine {
   bool tiles_ready_ = false;  // the latest re-sort built a work list, and it matches the layout
   uint64_t trail_elems_ = 0;
   // Captured chunks.  A chunk's launches depend on the current trail and
-  // agent buffers and on where the chunk starts in the re-sort schedule
-  // (absolute steps 0, k, 2k, ..., as eager steps follow), so that is the key.
+  // agent buffers, on where the chunk starts in the re-sort schedule
+  // (absolute steps 0, k, 2k, ..., as eager steps follow) and, where it does not
+  // start with a re-sort, on whether there is a work list: that is the key.
   struct ChunkKey {
     int cur, acur;
     uint32_t phase;  // steps_done % resort_interval at the chunk's start (0 without re-sorts)
+    bool tiles;      // tiles_ready_ at the chunk's start (false where it re-sorts first)
     bool operator==(const ChunkKey& o) const {
-      return cur == o.cur && acur == o.acur && phase == o.phase;
+      return cur == o.cur && acur == o.acur && phase == o.phase && tiles == o.tiles;
     }
   };
   static constexpr size_t kMaxCachedChunks = 16;  // per kind; the oldest goes first
@@ -1504,6 +1506,8 @@ class Engine {
       SLM_HIP(hipMemcpy(tile_inst_d_, tmap.data(), tmap.size() * 4ull, hipMemcpyHostToDevice));
       SLM_TRY(dev_alloc(&sort_.tile_items, total_tiles_ * 4ull));
       SLM_TRY(dev_alloc(&items_d_, max_items_ * sizeof(WorkItem)));
+      // an empty list until a re-sort has built one
+      SLM_HIP(hipMemsetAsync(items_d_, 0, max_items_ * sizeof(WorkItem), stream));
       uint32_t lv = plan_scan(sort_, total_bins_);
       SLM_TRY(dev_alloc(&scan_levels_, lv * 4ull));
       uint32_t at = 0;
@@ -1866,7 +1870,8 @@ class Engine {
   bool sorts_at(uint64_t step) const { return sort_due(step) && total_agents_ > 0; }
 
   ChunkKey chunk_key() const {
-    return {cur_, acur_, sorting() ? static_cast<uint32_t>(steps_done % cfg.resort_interval) : 0u};
+    const uint32_t phase = sorting() ? static_cast<uint32_t>(steps_done % cfg.resort_interval) : 0u;
+    return {cur_, acur_, phase, phase != 0u && tiles_ready_};
   }
 
   // Cached entry for `key` in `cache`, or nullptr.
@@ -1889,13 +1894,16 @@ class Engine {
         (void)hipGraphExecDestroy(graphs_.front().second);
         graphs_.erase(graphs_.begin());
       }
+      // nothing has run yet: the state is that of the steps before, whatever fails
       int cur0 = cur_, acur0 = acur_;
+      const bool tiles0 = tiles_ready_;
       hipGraph_t graph = nullptr;
       SLM_HIP(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
       enqueue_steps(s0, chunk);
       hipError_t e = hipStreamEndCapture(stream, &graph);
       cur_ = cur0;
       acur_ = acur0;
+      tiles_ready_ = tiles0;
       if (e != hipSuccess) return fail(SLM_ERR_HIP, "graph capture failed: %s", hipGetErrorString(e));
       e = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
       (void)hipGraphDestroy(graph);
@@ -1905,7 +1913,10 @@ class Engine {
     }
     SLM_HIP(hipGraphLaunch(exec, stream));
     for (uint32_t j = 0; j < chunk; j++) {  // the buffer swaps the captured steps make
-      if (sorts_at(s0 + j)) acur_ ^= 1;
+      if (sorts_at(s0 + j)) {
+        acur_ ^= 1;
+        tiles_ready_ = uses_tiles();
+      }
       cur_ ^= 1;
     }
     steps_done += chunk;

@@ -50,3 +50,27 @@ def test_choice_follows_the_steps_that_windows_serve(slm):
             assert sim.sensing() == 1
         sim.set_params(preset(slm, "Snake"))  # sensors that no window covers
         assert sim.sensing() == 0
+
+
+def test_replayed_chunks_lay_the_tiles_out(slm):
+    """A captured chunk that re-sorts leaves a work list behind each time it runs, also
+    after a snapshot was loaded; a chunk that starts between re-sorts uses it only where
+    it is there."""
+    kw = dict(seed=2, params=preset(slm, "Default"), resort_interval=20)
+    with slm.Simulation(1600, 900, 1 << 21, graph_chunk=10, **kw) as sim, \
+            slm.Simulation(1600, 900, 1 << 21, graph_chunk=0, **kw) as eager:
+        start = sim.snapshot()
+        sim.step(40)
+        sim.load_snapshot(start)
+        for steps in (10, 3):
+            sim.step(steps)
+            assert sim.sensing() == 1
+        eager.step(13)
+        middle = eager.snapshot()
+        assert sim.snapshot() == middle
+        sim.load_snapshot(middle)  # no list before the next re-sort, at step 20
+        assert sim.sensing() == 0
+        sim.step(10)  # one chunk, over the re-sort
+        assert sim.sensing() == 1
+        eager.step(10)
+        assert sim.snapshot() == eager.snapshot()
