@@ -498,6 +498,10 @@ class Engine {
     if (e == hipSuccess) {
       launch_unpack_agents(inst[k], agents_[acur_], pos64() ? 1 : 0,
                            static_cast<const float*>(st.p), stream);
+      // agents in their first order again, away from the tiles of the work list: once
+      // most of them are, windows would be staged that few read
+      rewritten_ += n;
+      if (rewritten_ * 2u > total_agents_) tiles_ready_ = false;
       e = hipStreamSynchronize(stream);
     }
     if (e != hipSuccess) return fail(SLM_ERR_HIP, "write_agents failed: %s", hipGetErrorString(e));
@@ -1167,7 +1171,9 @@ class Engine {
   uint32_t tile_steps_ = 0;             // tile_steps_now for them
   uint32_t* tile_inst_d_ = nullptr;
   WorkItem* items_d_ = nullptr;
-  bool tiles_ready_ = false;  // the latest re-sort built a work list, and it matches the layout
+  // the latest re-sort built a work list, and it matches the layout and most agents
+  bool tiles_ready_ = false;
+  uint64_t rewritten_ = 0;    // agents written since that re-sort
   uint64_t trail_elems_ = 0;
   // Captured chunks.  A chunk's launches depend on the current trail and
   // agent buffers, on where the chunk starts in the re-sort schedule
@@ -1630,10 +1636,16 @@ class Engine {
       launch_agents(p, agents_[acur_], trail_[cur_], stream);
   }
 
+  // A re-sort (just launched) has laid the agents out, and written a work list or not.
+  void resorted(bool list) {
+    tiles_ready_ = list;
+    rewritten_ = 0;
+  }
+
   void enqueue_sort(const Pool& p) {
     launch_morton_sort(p, agents_[acur_], agents_[acur_ ^ 1], sort_, stream);
     acur_ ^= 1;
-    tiles_ready_ = p.items != nullptr;
+    resorted(p.items != nullptr);
   }
 
   // Absolute step `step`; `between` runs after the agent pass is enqueued and
@@ -1897,6 +1909,7 @@ class Engine {
       // nothing has run yet: the state is that of the steps before, whatever fails
       int cur0 = cur_, acur0 = acur_;
       const bool tiles0 = tiles_ready_;
+      const uint64_t rewritten0 = rewritten_;
       hipGraph_t graph = nullptr;
       SLM_HIP(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
       enqueue_steps(s0, chunk);
@@ -1904,6 +1917,7 @@ class Engine {
       cur_ = cur0;
       acur_ = acur0;
       tiles_ready_ = tiles0;
+      rewritten_ = rewritten0;
       if (e != hipSuccess) return fail(SLM_ERR_HIP, "graph capture failed: %s", hipGetErrorString(e));
       e = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
       (void)hipGraphDestroy(graph);
@@ -1915,7 +1929,7 @@ class Engine {
     for (uint32_t j = 0; j < chunk; j++) {  // the buffer swaps the captured steps make
       if (sorts_at(s0 + j)) {
         acur_ ^= 1;
-        tiles_ready_ = uses_tiles();
+        resorted(uses_tiles());
       }
       cur_ ^= 1;
     }
@@ -2020,6 +2034,7 @@ class Engine {
     tc.sorted.assign(chunk, 0);
     const int cur0 = cur_, acur0 = acur_;
     const bool tiles0 = tiles_ready_;
+    const uint64_t rewritten0 = rewritten_;
     const Pool p = pool();
     hipGraph_t g = nullptr;
     hipError_t e = hipGraphCreate(&g, 0);
@@ -2065,6 +2080,7 @@ class Engine {
     cur_ = cur0;
     acur_ = acur0;
     tiles_ready_ = tiles0;
+    rewritten_ = rewritten0;
     if (e == hipSuccess) e = hipGraphInstantiate(&tc.exec, g, nullptr, nullptr, 0);
     if (g) (void)hipGraphDestroy(g);
     if (e != hipSuccess) {
@@ -2096,7 +2112,7 @@ class Engine {
     for (uint32_t j = 0; j < chunk; j++) {  // the buffer swaps the captured steps make
       if (tc.sorted[j]) {
         acur_ ^= 1;
-        tiles_ready_ = uses_tiles();
+        resorted(uses_tiles());
       }
       cur_ ^= 1;
     }

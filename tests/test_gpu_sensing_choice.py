@@ -74,3 +74,25 @@ def test_replayed_chunks_lay_the_tiles_out(slm):
         assert sim.sensing() == 1
         eager.step(10)
         assert sim.snapshot() == eager.snapshot()
+
+
+def test_written_agents_sense_from_global_memory_until_the_next_resort(slm):
+    """Agents written back stand in their first order, not in the work list's tiles."""
+    kw = dict(seed=2, params=preset(slm, "Default"), resort_interval=20, graph_chunk=0)
+    with slm.Simulation(1600, 900, 1 << 21, **kw) as sim:
+        sim.step(3)
+        a = sim.read_agents()
+        assert sim.sensing() == 1
+        sim.write_agents(a)
+        assert sim.sensing() == 0
+        sim.step(17)
+        assert sim.sensing() == 1  # step 20 re-sorts
+        sim.step(1)
+        assert sim.sensing() == 1
+    with slm.Batch([slm.InstanceSpec(512, 512, 1 << 18, seed=k, params=preset(slm, "Default"))
+                    for k in range(9)], resort_interval=20, graph_chunk=0) as b:
+        b.step(1)
+        for k in range(5):  # windows serve the others while these are most agents
+            assert b.sensing() == 1
+            b.write_agents(k, b.read_agents(k))
+        assert b.sensing() == 0
