@@ -203,10 +203,10 @@ int slm_destroy(slm_sim* sim);
 /* Replace the parameters for subsequent steps; agents and trail persist.
  * Replaces update_settings / the preset switch (src/main.rs:83-99, :815-832).
  * Captured graphs stay valid: kernels read parameters from device memory.
- * Two exceptions.  Where the library senses through tile windows (see
- * SLM_FLAG_TILED_SENSING), a change of sensor distance or speeds that changes how
- * many steps after a re-sort the windows fit drops the captured graphs likewise.
- * And with SLM_FLAG_GAUSSIAN_DIFFUSE: a 16-bit pool's Gaussian pass
+ * (Where the library senses through tile windows, see SLM_FLAG_TILED_SENSING, and a
+ * change of sensor distance or speeds changes how many steps after a re-sort they
+ * fit, the second chunk of steps under the new parameters is captured anew.)
+ * One exception, with SLM_FLAG_GAUSSIAN_DIFFUSE: a 16-bit pool's Gaussian pass
  * sizes its LDS tile (and its tile height) for the largest radius class
  * (R <= 2, <= 4, <= 8) of its instances, so a change of class waits for the
  * handle's stream, drops the captured graphs (the next slm_step recaptures

@@ -11,7 +11,8 @@
 // plus re-sort scratch, f64 mass scratch and one non-blocking HIP stream.
 // Steps are enqueued eagerly or as captured hipGraphs of `graph_chunk` steps;
 // a graph is keyed by which trail and agent buffers are current when it
-// starts, so at most four exist per handle.  Every entry point validates its
+// starts, where in the re-sort schedule that is and how its steps sense, and at
+// most kMaxCachedChunks are kept per handle.  Every entry point validates its
 // arguments before any kernel is launched, so the kernels can rely on
 // in-range shapes and finite, bounded positions.
 #include <algorithm>
@@ -440,18 +441,12 @@ class Engine {
         if (replan) return relayout(layout_trail_tables());
       }
     }
-    // captured chunks hold the sensing of the parameters they were captured under
-    // (their results hold for any): recapture where another one pays
     const uint32_t fits = auto_tiles() ? window_steps(k) : 0u;
     if (fits != window_steps_[k]) {
       window_steps_[k] = fits;
-      const uint32_t tiles = tile_steps_now();
-      if (tiles != tile_steps_) {
-        SLM_HIP(hipStreamSynchronize(stream));
-        drop_graphs();
-        tile_steps_ = tiles;
-      }
+      tile_steps_known_ = false;
     }
+    params_moved_ = true;
     return SLM_OK;
   }
 
@@ -1168,7 +1163,8 @@ class Engine {
   uint64_t total_cells_ = 0;
   double window_tiles_ = 1;  // 64 x 64-cell tiles that reach into the instances' grids
   std::vector<uint32_t> window_steps_;  // per instance, for the current layout and parameters
-  uint32_t tile_steps_ = 0;             // tile_steps_now for them
+  mutable uint32_t tile_steps_ = 0;     // tile_steps() for them, once known
+  mutable bool tile_steps_known_ = false;
   uint32_t* tile_inst_d_ = nullptr;
   WorkItem* items_d_ = nullptr;
   // the latest re-sort built a work list, and it matches the layout and most agents
@@ -1178,15 +1174,24 @@ class Engine {
   // Captured chunks.  A chunk's launches depend on the current trail and
   // agent buffers, on where the chunk starts in the re-sort schedule
   // (absolute steps 0, k, 2k, ..., as eager steps follow) and, where it does not
-  // start with a re-sort, on whether there is a work list: that is the key.
+  // start with a re-sort, on whether there is a work list; and which steps sense
+  // through windows on tile_steps(): that is the key.
   struct ChunkKey {
     int cur, acur;
     uint32_t phase;  // steps_done % resort_interval at the chunk's start (0 without re-sorts)
     bool tiles;      // tiles_ready_ at the chunk's start (false where it re-sorts first)
-    bool operator==(const ChunkKey& o) const {
+    uint32_t tile_steps;
+    bool same_state(const ChunkKey& o) const {
       return cur == o.cur && acur == o.acur && phase == o.phase && tiles == o.tiles;
     }
+    bool operator==(const ChunkKey& o) const { return same_state(o) && tile_steps == o.tile_steps; }
   };
+  // Parameters were set since the last captured chunk ran.  They may have moved
+  // tile_steps(), but a chunk's results hold for any: the first chunk after them replays
+  // one captured under others where there is one (its windows fit better or worse), so
+  // that a program which moves a parameter before every chunk captures none, and the
+  // second, if they stay, captures its own.
+  bool params_moved_ = false;
   static constexpr size_t kMaxCachedChunks = 16;  // per kind; the oldest goes first
   std::vector<std::pair<ChunkKey, hipGraphExec_t>> graphs_;
   std::vector<std::pair<void*, size_t>> allocs_;
@@ -1467,7 +1472,7 @@ class Engine {
     window_steps_.assign(spec.size(), 0u);
     if (auto_tiles())
       for (size_t k = 0; k < spec.size(); k++) window_steps_[k] = window_steps(k);
-    tile_steps_ = tile_steps_now();
+    tile_steps_known_ = false;
 
     dev_free(unit_block_d_);
     uint32_t nb = blocks_for(units, kTrailWavesPerBlock);
@@ -1545,8 +1550,11 @@ class Engine {
     return static_cast<uint64_t>(max_items_) * tile_block(pos64()) < (1ull << 32);
   }
 
-  // Whether any step senses through tile windows.
-  bool uses_tiles() const { return (cfg.flags & SLM_FLAG_TILED_SENSING) || tile_steps_ > 0u; }
+  // Whether any step senses through tile windows, where they serve tile_steps steps.
+  bool uses_tiles(uint32_t tile_steps) const {
+    return (cfg.flags & SLM_FLAG_TILED_SENSING) || tile_steps > 0u;
+  }
+  bool uses_tiles() const { return uses_tiles(tile_steps()); }
 
   // Whether the pool's agents sense through tile windows of the library's own
   // accord: with the plain re-sort key, one launch per pass over the pool and no
@@ -1598,10 +1606,15 @@ class Engine {
   // through windows; 0 where the pool does not.  Building the work list is six more
   // launches of about 3 us at each re-sort, and windows save about 2 us a step for
   // each 2^20 agents: they are taken where the steps they serve win that back.
-  uint32_t tile_steps_now() const {
+  // Found when it is next asked for: a program may set every instance's parameters.
+  uint32_t tile_steps() const {
     constexpr uint64_t kMinAgentSteps = 10u << 20;
-    const uint32_t steps = auto_tiles() ? half_window_steps() : 0u;
-    return static_cast<uint64_t>(steps) * total_agents_ >= kMinAgentSteps ? steps : 0u;
+    if (!tile_steps_known_) {
+      const uint32_t steps = auto_tiles() ? half_window_steps() : 0u;
+      tile_steps_ = static_cast<uint64_t>(steps) * total_agents_ >= kMinAgentSteps ? steps : 0u;
+      tile_steps_known_ = true;
+    }
+    return tile_steps_;
   }
   uint32_t half_window_steps() const {
     std::vector<std::pair<uint32_t, uint64_t>> by_steps;
@@ -1623,7 +1636,7 @@ class Engine {
   // Whether that step senses through tile windows, with (ready) a work list or without.
   bool senses_tiles(uint64_t step, bool ready) const {
     return sorting() && ready && tiles_launchable() &&
-           ((cfg.flags & SLM_FLAG_TILED_SENSING) || drift_at(step) <= tile_steps_);
+           ((cfg.flags & SLM_FLAG_TILED_SENSING) || drift_at(step) <= tile_steps());
   }
 
   // Tiled sensing (when asked for, or where it pays: auto_tiles) once a re-sort
@@ -1883,7 +1896,7 @@ class Engine {
 
   ChunkKey chunk_key() const {
     const uint32_t phase = sorting() ? static_cast<uint32_t>(steps_done % cfg.resort_interval) : 0u;
-    return {cur_, acur_, phase, phase != 0u && tiles_ready_};
+    return {cur_, acur_, phase, phase != 0u && tiles_ready_, tile_steps()};
   }
 
   // Cached entry for `key` in `cache`, or nullptr.
@@ -1897,9 +1910,16 @@ class Engine {
   int run_chunk_graph() {
     const uint32_t chunk = cfg.graph_chunk;
     const uint64_t s0 = steps_done;
-    const ChunkKey key = chunk_key();
-    hipGraphExec_t* found = cached(graphs_, key);
-    hipGraphExec_t exec = found ? *found : nullptr;
+    ChunkKey key = chunk_key();
+    hipGraphExec_t exec = nullptr;
+    for (auto& e : graphs_)
+      if (e.first == key) exec = e.second;
+    if (!exec && params_moved_)
+      for (auto& e : graphs_)
+        if (e.first.same_state(key)) {
+          key = e.first;
+          exec = e.second;
+        }
     if (!exec) {
       if (graphs_.size() >= kMaxCachedChunks) {  // drop the oldest, once it has run
         SLM_HIP(hipStreamSynchronize(stream));
@@ -1929,11 +1949,12 @@ class Engine {
     for (uint32_t j = 0; j < chunk; j++) {  // the buffer swaps the captured steps make
       if (sorts_at(s0 + j)) {
         acur_ ^= 1;
-        resorted(uses_tiles());
+        resorted(uses_tiles(key.tile_steps));  // as it was captured
       }
       cur_ ^= 1;
     }
     steps_done += chunk;
+    params_moved_ = false;
     return SLM_OK;
   }
 

@@ -96,3 +96,44 @@ def test_written_agents_sense_from_global_memory_until_the_next_resort(slm):
             assert b.sensing() == 1
             b.write_agents(k, b.read_agents(k))
         assert b.sensing() == 0
+
+
+def test_parameters_moved_before_every_chunk(slm, orc):
+    """Speeds that change how long the windows fit, set before every captured chunk of
+    steps, and then left for some: the same bits as the unsorted run."""
+    import dataclasses
+    base = preset(slm, "Default")
+    speeds = [base.agent_speed_max, 400.0, 90.0, 1500.0, 90.0, 90.0, 90.0, 5000.0, 60.0, 60.0]
+    out = []
+    for kw in (dict(), dict(resort_interval=12, graph_chunk=6)):
+        with slm.Simulation(1600, 900, 1 << 21, seed=5, params=base, **kw) as sim:
+            for k, v in enumerate(speeds):
+                sim.set_params(dataclasses.replace(base, agent_speed_max=v, agent_speed_min=v / 2))
+                sim.step(6 if k % 3 else 12)
+            sim.step(2)
+            out.append((sim.read_agents(), sim.read_trail()))
+    assert_bitwise(out[1][0], out[0][0], "agents")
+    assert_bitwise(out[1][1], out[0][1], "trail")
+
+
+def test_parameters_are_set_without_waiting(slm):
+    """slm_set_params returns while earlier steps still run, also where it changes how
+    long the windows fit."""
+    import dataclasses
+    import time
+    base = preset(slm, "Default")
+    fast = dataclasses.replace(base, agent_speed_max=900.0)
+    with slm.Simulation(4096, 4096, 1 << 24, seed=5, params=base, resort_interval=20,
+                        graph_chunk=20) as sim:
+        for s in (base, fast, base, fast):  # both captured
+            sim.set_params(s)
+            sim.step(80)
+        sim.synchronize()
+        t0 = time.perf_counter()
+        sim.step(400)
+        sim.set_params(base)
+        returned = time.perf_counter() - t0
+        sim.synchronize()
+        total = time.perf_counter() - t0
+    print(f"[set_params] returned after {returned * 1e3:.2f} of {total * 1e3:.2f} ms", flush=True)
+    assert returned < 0.5 * total
