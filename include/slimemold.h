@@ -324,13 +324,15 @@ typedef struct slm_tuning {
   uint32_t resort_interval;  /* Morton re-sort of agents every k steps; 0 = never */
   uint32_t sort_cell_log2;   /* re-sort bin edge = 2^k cells, k <= 12 */
   uint32_t agents_per_group; /* agents one workgroup of the agent pass updates:
-                                256, 512, 1024, 2048 or 4096 */
+                                256, 512, 1024, 2048 or 4096 (tile windows have
+                                their own workgroups) */
   uint32_t trail_rows;       /* rows of one trail-pass tile (64*vector-width
                                 columns): 4, 8, 16, 32 or 64; 0 = the library's
                                 choice (4) */
   uint32_t tiled_sensing;    /* 1 = SLM_FLAG_TILED_SENSING (needs re-sorting),
-                                2 = SLM_FLAG_WINDOW_SENSING, 0 = the library's
-                                choice of global memory or tile windows */
+                                2 = SLM_FLAG_WINDOW_SENSING, SLM_SENSING_GLOBAL =
+                                global memory, 0 = the library's choice of
+                                global memory or tile windows */
   uint32_t trials;           /* autotune: configurations timed; else 0 */
   uint32_t instance_groups;  /* 1..4096 (0 reads as 1): between re-sorts the
                                 instances step as this many contiguous groups
@@ -363,6 +365,7 @@ typedef struct slm_tuning {
   double step_ms, agents_ms, trail_ms, sort_ms;
 } slm_tuning;
 
+#define SLM_SENSING_GLOBAL 4u
 #define SLM_SORT_HEADING_MASK 0x7u
 #define SLM_SORT_AT_SENSOR 0x10u
 
@@ -378,7 +381,7 @@ int slm_set_tuning(slm_sim* sim, const slm_tuning* tuning);
 /* Times candidate tunings on the simulation's own state and keeps the
  * fastest: the trail tile rows by trail-pass time, streaming (0..3), then the
  * re-sort interval
- * (0, 5, 10, 20 or 40), the bin size, the sensing mode (0, 1, 2), agents per workgroup and
+ * (0, 5, 10, 20 or 40), the bin size, the sensing mode, agents per workgroup and
  * (batches) instance groups (powers of 4 up to the instance count, then the
  * best one's neighbours x2 and /2) by total step time (coordinate descent).
  * Step times are spans over steps launched as slm_step launches them; kernel

@@ -166,6 +166,7 @@ struct EngineConfig {
   uint32_t instance_groups = 1;
   uint32_t streaming = 0;
   uint32_t sort_key = 0;  // SLM_SORT_* refinement of the re-sort key
+  bool global_sensing = false;  // SLM_SENSING_GLOBAL: no tile windows of the library's own accord
 };
 
 constexpr uint32_t kMaxInstanceGroups = 4096;
@@ -179,7 +180,8 @@ int check_tuning(const slm_tuning& t) {
   uint32_t r = t.trail_rows;
   if (r != 0 && (r < 4 || r > 64 || (r & (r - 1u))))
     return fail(SLM_ERR_INVALID_ARGUMENT, "trail_rows must be 0, 4, 8, 16, 32 or 64");
-  if (t.tiled_sensing > 2) return fail(SLM_ERR_INVALID_ARGUMENT, "tiled_sensing must be 0, 1 or 2");
+  if (t.tiled_sensing > 2 && t.tiled_sensing != SLM_SENSING_GLOBAL)
+    return fail(SLM_ERR_INVALID_ARGUMENT, "tiled_sensing must be 0, 1, 2 or SLM_SENSING_GLOBAL");
   if (t.instance_groups > kMaxInstanceGroups)
     return fail(SLM_ERR_INVALID_ARGUMENT, "instance_groups must be <= %u", kMaxInstanceGroups);
   if (t.streaming > 3) return fail(SLM_ERR_INVALID_ARGUMENT, "streaming must be 0..3");
@@ -748,6 +750,7 @@ class Engine {
     t.trail_rows = cfg.trail_rows;
     t.tiled_sensing = (cfg.flags & SLM_FLAG_TILED_SENSING)   ? 1u
                       : (cfg.flags & SLM_FLAG_WINDOW_SENSING) ? 2u
+                      : cfg.global_sensing                    ? SLM_SENSING_GLOBAL
                                                               : 0u;
     t.instance_groups = cfg.instance_groups;
     t.streaming = cfg.streaming;
@@ -949,6 +952,7 @@ class Engine {
       cfg.flags &= ~(SLM_FLAG_TILED_SENSING | SLM_FLAG_WINDOW_SENSING);
       if (t.tiled_sensing == 1) cfg.flags |= SLM_FLAG_TILED_SENSING;
       if (t.tiled_sensing == 2) cfg.flags |= SLM_FLAG_WINDOW_SENSING;
+      cfg.global_sensing = t.tiled_sensing == SLM_SENSING_GLOBAL;
       if (new_agents) SLM_TRY(layout_agents());
       return layout_trail_tables();
     }());
@@ -1079,13 +1083,18 @@ class Engine {
         SLM_TRY(take(t));
       }
     }
-    // sensing: global taps (0), tile work lists (1: needs re-sorting with the
-    // plain key and one instance group), per-workgroup LDS windows (2)
+    // sensing: the library's choice (0), tile windows always (1: needs re-sorting with
+    // the plain key and one instance group), per-workgroup LDS windows (2), global
+    // memory only.  Of 0 and its equal here, global memory where the library would not
+    // choose windows and windows where it would, one is enough.
     {
       const uint32_t cur = best.tiled_sensing;
-      for (uint32_t m : {0u, 1u, 2u}) {
-        if (m == cur || (m == 1u && (!best.resort_interval || best.instance_groups > 1 ||
-                                     best.sort_key != 0u)))
+      const bool chosen = windows_pay(best.resort_interval, best.instance_groups, best.sort_key);
+      for (uint32_t m : {0u, 1u, 2u, SLM_SENSING_GLOBAL}) {
+        if (m == cur || m == (chosen ? 1u : SLM_SENSING_GLOBAL) ||
+            (m == 1u && (!best.resort_interval || best.instance_groups > 1 ||
+                         best.sort_key != 0u)) ||
+            (m == 0u && !chosen && cur == SLM_SENSING_GLOBAL))
           continue;
         slm_tuning t = best;
         t.tiled_sensing = m;
@@ -1571,14 +1580,17 @@ class Engine {
   //     2048    one 2048^2 0.86, 1024 of 64^2 0.91 (f64 0.85, 1.0)
   //     4096    one 2048^2 0.75, one 4096^2 0.68, 512 of 64^2 0.83
   bool auto_tiles() const {
+    return !cfg.global_sensing && !(cfg.flags & SLM_FLAG_WINDOW_SENSING) &&
+           windows_pay(cfg.resort_interval, cfg.instance_groups, cfg.sort_key);
+  }
+  bool windows_pay(uint32_t resort_interval, uint32_t instance_groups, uint32_t sort_key) const {
     const uint64_t min_agents = pos64() ? 1u << 22 : 1u << 21;
     const double min_per_tile = pos64() ? 1900.0 : 1550.0;
     constexpr double kTileCells = double(1u << (2 * kTileLog2));
     const double per_tile = static_cast<double>(total_agents_) / window_tiles_ *
                             (static_cast<double>(total_cells_) / (window_tiles_ * kTileCells));
-    return sorting() && groups_.size() <= 1 && cfg.sort_key == 0u &&
-           !(cfg.flags & (SLM_FLAG_WINDOW_SENSING | SLM_FLAG_PERSISTENT)) &&
-           total_agents_ >= min_agents && per_tile >= min_per_tile;
+    return resort_interval > 0 && std::min(instance_groups, count()) <= 1 && sort_key == 0u &&
+           !(cfg.flags & SLM_FLAG_PERSISTENT) && total_agents_ >= min_agents && per_tile >= min_per_tile;
   }
 
   // The most steps after a re-sort, up to the interval, at which instance k's tile

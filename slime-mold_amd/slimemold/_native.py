@@ -32,6 +32,7 @@ FLAG_WINDOW_SENSING = 0x20
 FLAG_PERSISTENT = 0x40
 SORT_HEADING_MASK = 0x7
 SORT_AT_SENSOR = 0x10
+SENSING_GLOBAL = 4
 
 
 class NativeLibraryMissing(RuntimeError):

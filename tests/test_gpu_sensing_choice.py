@@ -137,3 +137,26 @@ def test_parameters_are_set_without_waiting(slm):
         total = time.perf_counter() - t0
     print(f"[set_params] returned after {returned * 1e3:.2f} of {total * 1e3:.2f} ms", flush=True)
     assert returned < 0.5 * total
+
+
+def test_global_sensing_can_be_asked_for(slm):
+    kw = dict(seed=4, params=preset(slm, "Default"), resort_interval=10)
+    with slm.Simulation(1600, 900, 1 << 21, **kw) as sim, \
+            slm.Simulation(1600, 900, 1 << 21, **kw) as ref:
+        sim.set_tuning(tiled_sensing=4)
+        assert sim.get_tuning().tiled_sensing == 4 and sim.sensing() == 0
+        sim.step(13)
+        assert sim.sensing() == 0
+        sim.set_tuning(trail_rows=8)  # kept
+        assert sim.get_tuning().tiled_sensing == 4 and sim.sensing() == 0
+        sim.set_tuning(tiled_sensing=0)
+        assert sim.sensing() == 0  # until a re-sort writes the list
+        sim.step(7)
+        assert sim.sensing() == 1
+        ref.step(20)
+        assert sim.snapshot() == ref.snapshot()
+        chosen = sim.autotune(trial_steps=40)
+        print(f"[global sensing] {chosen.as_dict()}", flush=True)
+        sim.step(5)
+        ref.step(5)
+        assert sim.snapshot() == ref.snapshot()
