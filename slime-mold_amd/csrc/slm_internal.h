@@ -353,8 +353,17 @@ void launch_unpack_positions64(const Instance& in, const AgentSoA& a, const doub
                                hipStream_t stream);
 
 // ---- Morton re-sort ------------------------------------------------------
+// Pools up to this many agents re-sort by a rank per agent: the count kernel writes each
+// agent's rank in its bin, and the scatter is one load and store.  Larger ones reserve
+// runs of slots and order their agents in LDS (scatter_kernel).  The short form wins
+// where latency counts, the other where its stores do, in us per re-sort, short / LDS:
+// 2^14 agents on 256^2 16.3 / 19.6, 2^18 on 1024^2 22.9 / 25.1, 2^21 on 2048^2 41.7 /
+// 44.9, 2^22 on 256^2 57.5 / 60.5, 2048^2 61.9 / 66.0, 4096^2 78 / 71, 2^23 on 2048^2
+// 126 / 116; with f64 positions 2^20 on 1024^2 34.4 / 34.5, 2^22 89 / 79.
+constexpr uint64_t ranked_agents(bool pos64) { return pos64 ? 1u << 21 : 1u << 22; }
 struct SortScratch {
-  uint32_t* count;     // per bin: agents, then those still to be scattered
+  uint32_t* rank;      // per slot: rank inside its bin; nullptr beyond ranked_agents
+  uint32_t* count;     // per bin: agents, then (no rank) those still to be scattered
   uint32_t* offset;    // per bin, exclusive prefix sum; offset[total_bins] = total agents
   uint32_t* tile_items;  // per tile: work items, then their exclusive prefix sum
   uint32_t* level[3];  // tile sums of the multi-level scan

@@ -76,8 +76,10 @@ __global__ void zero_u32_kernel(uint32_t* p, uint32_t n) {
 // is its key mod kLocalBins: the Morton codes of any 32 x 32 bins differ in their low
 // 10 bits, also where the region straddles an edge of a large aligned square and
 // its codes lie far apart (a table by distance from the lowest code refuses those,
-// a quarter of the workgroups or more).  Where two bins meet in an entry the
-// workgroup falls back to atomics on the global counters.
+// a quarter of the workgroups or more).  Where two bins meet in an entry one of them
+// has it, and the other's agents take atomics on the global counters (all agents of
+// such a workgroup did: where one instance's last agents wrap to its first bins, beside
+// the next one's, 350 instances of 40 x 300 with 2.1 * 10^6 agents counted in 25 us).
 constexpr uint32_t kLocalBins = 1024;  // LDS for 5 workgroups a CU (2048: 4, up to 7% slower)
 constexpr int kSortPer = 4;
 constexpr uint32_t kSortSlots = kSortPer * kAgentBlock;
@@ -105,13 +107,11 @@ __device__ inline bool sort_slot(const SortArgs& g, uint32_t base, int q, uint32
   return uint64_t(base) + q * kAgentBlock + threadIdx.x < g.total;
 }
 
-// The keys of the workgroup's agents, their ranks among its agents of the bin, and
-// whether each bin has an entry of its own in `s_cnt`, which then holds the bin's
-// agents (uniform).  s_tag is scratch, free again on return.
+// The keys of the workgroup's agents, whether their bin has its entry, with the bin's
+// agents here in `s_cnt` and its key in `s_tag`, and then their ranks among them.
 struct Keys {
   uint32_t k[kSortPer], r[kSortPer];
-  bool act[kSortPer];
-  bool local;
+  bool act[kSortPer], own[kSortPer];
   __device__ uint32_t entry(int q) const { return k[q] & (kLocalBins - 1u); }
 };
 __device__ inline Keys block_keys(const SortArgs& g, uint32_t base, const float (&x)[kSortPer],
@@ -123,6 +123,7 @@ __device__ inline Keys block_keys(const SortArgs& g, uint32_t base, const float 
   for (int q = 0; q < kSortPer; q++) {
     uint32_t j;
     t.act[q] = sort_slot(g, base, q, j);
+    t.own[q] = false;
     t.k[q] = t.r[q] = 0;
   }
 #pragma unroll
@@ -143,19 +144,38 @@ __device__ inline Keys block_keys(const SortArgs& g, uint32_t base, const float 
   for (int q = 0; q < kSortPer; q++)
     if (t.act[q]) s_tag[t.entry(q)] = t.k[q];
   __syncthreads();
-  bool shared = false;
 #pragma unroll
   for (int q = 0; q < kSortPer; q++)
-    if (t.act[q]) {
-      shared |= s_tag[t.entry(q)] != t.k[q];
+    if (t.act[q] && s_tag[t.entry(q)] == t.k[q]) {
+      t.own[q] = true;
       t.r[q] = atomicAdd(&s_cnt[t.entry(q)], 1u);
     }
-  t.local = !__syncthreads_or(shared);
+  __syncthreads();
   return t;
 }
 
-// The fallback: old = add(bin, n) by one lane for n lanes of a wave in the bin, then
-// use(q, old, rank among them) by each.  The first few distinct bins of a wave are
+// s_tag[entry] = add(bin, its agents) for each bin that has its entry: entry by entry, so
+// that neighbouring bins' counters are reached by neighbouring lanes, and all in flight
+// before one is used.  (One lane per bin wherever its first agent stood: count and
+// scatter of 2^24 agents on 4096^2 230 us instead of 209, on 256^2 with 8 * 10^6
+// agents 129 instead of 112.)
+template <class Add>
+__device__ inline void each_bin(const uint32_t* s_cnt, uint32_t* s_tag, Add&& add) {
+  constexpr uint32_t kPer = kLocalBins / kAgentBlock;
+  uint32_t n[kPer], old[kPer];
+#pragma unroll
+  for (uint32_t i = 0; i < kPer; i++) {
+    const uint32_t e = i * kAgentBlock + threadIdx.x;
+    n[i] = s_cnt[e];
+    old[i] = n[i] ? add(s_tag[e], n[i]) : 0u;
+  }
+#pragma unroll
+  for (uint32_t i = 0; i < kPer; i++)
+    if (n[i]) s_tag[i * kAgentBlock + threadIdx.x] = old[i];
+}
+
+// The agents without an entry: old = add(bin, n) by one lane for n lanes of a wave in
+// the bin, then use(q, old, rank among them) by each.  The first few distinct bins of a wave are
 // taken together (agents that crowd a few distant bins), the others lane by lane
 // (agents in any order, as before the first re-sort, share almost none).
 constexpr int kWaveBins = 4;
@@ -164,7 +184,7 @@ __device__ inline void each_wave_bin(const Keys& t, Add&& add, Use&& use) {
   const int lane = static_cast<int>(threadIdx.x & 63u);
 #pragma unroll
   for (int q = 0; q < kSortPer; q++) {
-    bool todo = t.act[q];
+    bool todo = t.act[q] && !t.own[q];
     for (int n = 0; n < kWaveBins; n++) {
       const uint64_t pending = __ballot(todo);
       if (!pending) break;
@@ -181,11 +201,12 @@ __device__ inline void each_wave_bin(const Keys& t, Add&& add, Use&& use) {
   }
 }
 
-// count[bin] += the bin's agents.  All of a thread's agents are loaded before any
-// is used: with one agent per thread the chain of load, barrier and atomic per
-// block set the kernel's time, not the bandwidth.
+// count[bin] += the bin's agents; kRank: rank[slot] = the agent's rank in its bin.  All
+// of a thread's agents are loaded before any is used: with one agent per thread the
+// chain of load, barrier and atomic per block set the kernel's time, not the bandwidth.
+template <bool kRank>
 __global__ __launch_bounds__(kAgentBlock) void count_kernel(SortArgs g, AgentSoA a, int pos64,
-                                                            uint32_t* count) {
+                                                            uint32_t* count, uint32_t* rank) {
   __shared__ uint32_t s_cnt[kLocalBins], s_tag[kLocalBins];
   const uint32_t base = sort_base(g);
   float px[kSortPer], py[kSortPer], pth[kSortPer];
@@ -202,15 +223,17 @@ __global__ __launch_bounds__(kAgentBlock) void count_kernel(SortArgs g, AgentSoA
     }
   }
   const Keys t = block_keys(g, base, px, py, pth, s_cnt, s_tag);
-  if (!t.local) {
-    each_wave_bin(
-        t, [&](uint32_t k, uint32_t n) { return atomicAdd(count + k, n); },
-        [](int, uint32_t, uint32_t) {});
-    return;
-  }
+  auto add = [&](uint32_t k, uint32_t n) { return atomicAdd(count + k, n); };
+  each_bin(s_cnt, s_tag, add);
+  each_wave_bin(t, add, [&](int q, uint32_t first, uint32_t r) {
+    if constexpr (kRank) rank[base + q * kAgentBlock + threadIdx.x] = first + r;
+  });
+  if constexpr (kRank) {
+    __syncthreads();
 #pragma unroll
-  for (int q = 0; q < kSortPer; q++)  // by the first agent of each bin
-    if (t.act[q] && t.r[q] == 0u) atomicAdd(count + t.k[q], s_cnt[t.entry(q)]);
+    for (int q = 0; q < kSortPer; q++)
+      if (t.own[q]) rank[base + q * kAgentBlock + threadIdx.x] = s_tag[t.entry(q)] + t.r[q];
+  }
 }
 
 // Exclusive scan of one tile of `in` into `out` (in place allowed); writes
@@ -259,10 +282,10 @@ __global__ __launch_bounds__(kScanBlock) void scan_add_kernel(uint32_t* out, uin
 //
 // The vector L1 takes a divergent store one lane a cycle, so writing each agent
 // where it goes costs 64 accesses per array and wave (count and scatter of 2^24
-// agents, f32: 117 + 230 us).  The workgroup orders its agents by bin in LDS
+// agents, f32: 111 + 214 us).  The workgroup orders its agents by bin in LDS
 // instead (each bin's agents are reserved one run of slots) and writes the runs:
-// 52 + 190 us; 8192^2 bf16 with f64 positions and 2^26 agents 443 + 930 -> 288 + 777;
-// 64 instances of 256^2 to 2048^2 with 5 * 10^7 agents 516 + 716 -> 160 + 670.
+// 50 + 151 us; 8192^2 bf16 with f64 positions and 2^26 agents 398 + 831 -> 282 + 701;
+// 64 instances of 256^2 to 2048^2 with 5 * 10^7 agents 480 + 692 -> 134 + 449.
 // Bound by the LDS passes and the reservation's round trip.
 template <bool P64>
 __global__ __launch_bounds__(kAgentBlock) void scatter_kernel(SortArgs g, AgentSoA src,
@@ -305,21 +328,16 @@ __global__ __launch_bounds__(kAgentBlock) void scatter_kernel(SortArgs g, AgentS
   const Keys t = block_keys(g, base, fx, fy, th, s_cnt, s_base);
   // the first of n slots for agents of bin k
   auto reserve = [&](uint32_t k, uint32_t n) { return offset[k] + atomicSub(count + k, n) - n; };
-  if (!t.local) {
-    each_wave_bin(t, reserve, [&](int q, uint32_t first, uint32_t rank) {
-      const uint32_t d = first + rank;
-      if (d >= g.total) return;  // unreachable: the count kernel's bins
-      dx[d] = x[q];
-      dy[d] = y[q];
-      dst.th[d] = th[q];
-      dst.v[d] = v[q];
-      dst.id[d] = id[q];
-    });
-    return;
-  }
-#pragma unroll
-  for (int q = 0; q < kSortPer; q++)  // by the first agent of each bin
-    if (t.act[q] && t.r[q] == 0u) s_base[t.entry(q)] = reserve(t.k[q], s_cnt[t.entry(q)]);
+  each_bin(s_cnt, s_base, reserve);
+  each_wave_bin(t, reserve, [&](int q, uint32_t first, uint32_t rank) {
+    const uint32_t d = first + rank;
+    if (d >= g.total) return;  // unreachable: the count kernel's bins
+    dx[d] = x[q];
+    dy[d] = y[q];
+    dst.th[d] = th[q];
+    dst.v[d] = v[q];
+    dst.id[d] = id[q];
+  });
   // each bin's first position: thread i scans kPer consecutive bins
   constexpr uint32_t kPer = kLocalBins / kAgentBlock;
   const uint32_t lane = threadIdx.x & 63u;
@@ -338,7 +356,12 @@ __global__ __launch_bounds__(kAgentBlock) void scatter_kernel(SortArgs g, AgentS
   if (lane == 63u) s_dst[threadIdx.x >> 6] = run;
   __syncthreads();
   run -= sum;
-  for (uint32_t i = 0; i < threadIdx.x >> 6; i++) run += s_dst[i];
+  uint32_t placed = 0;  // the workgroup's agents with an entry
+#pragma unroll
+  for (uint32_t i = 0; i < kAgentBlock / 64; i++) {
+    if (i < threadIdx.x >> 6) run += s_dst[i];
+    placed += s_dst[i];
+  }
 #pragma unroll
   for (uint32_t i = 0; i < kPer; i++) {
     s_cnt[threadIdx.x * kPer + i] = run;
@@ -347,7 +370,7 @@ __global__ __launch_bounds__(kAgentBlock) void scatter_kernel(SortArgs g, AgentS
   __syncthreads();
 #pragma unroll
   for (int q = 0; q < kSortPer; q++)
-    if (t.act[q]) {
+    if (t.own[q]) {
       const uint32_t p = s_cnt[t.entry(q)] + t.r[q];
       s_dst[p] = s_base[t.entry(q)] + t.r[q];
       s_x[p] = x[q];
@@ -360,7 +383,7 @@ __global__ __launch_bounds__(kAgentBlock) void scatter_kernel(SortArgs g, AgentS
 #pragma unroll
   for (int q = 0; q < kSortPer; q++) {
     const uint32_t p = q * kAgentBlock + threadIdx.x;
-    if (!t.act[q]) continue;  // the workgroup's n agents hold positions 0 .. n - 1
+    if (p >= placed) continue;
     const uint32_t d = s_dst[p];
     if (d >= g.total) continue;  // unreachable: the count kernel's bins
     dx[d] = s_x[p];
@@ -369,6 +392,56 @@ __global__ __launch_bounds__(kAgentBlock) void scatter_kernel(SortArgs g, AgentS
     dst.v[d] = __uint_as_float(s_v[p]);
     dst.id[d] = s_id[p];
   }
+}
+
+// The scatter of pools up to ranked_agents: each agent straight to offset[bin] + rank,
+// its bin recomputed by the count kernel's arithmetic.  No barrier and no atomic: a load
+// and a store, in workgroups of kAgentBlock slots.  (Speed and index are loaded where they
+// are stored: loaded with the others, 2^22 agents on 256^2 take 58.5 us instead of 57.5.)
+template <bool P64>
+__global__ __launch_bounds__(kAgentBlock) void scatter_ranked_kernel(
+    SortArgs g, AgentSoA src, AgentSoA dst, const uint32_t* rank, const uint32_t* offset) {
+  const uint32_t blk = g.xcd_remap ? xcd_logical_block(blockIdx.x, gridDim.x) : blockIdx.x;
+  const uint32_t first = blk * kAgentBlock, last = min(first + kAgentBlock, g.total) - 1u;
+  const uint32_t j = first + threadIdx.x;
+  const bool act = j < g.total;
+  double x64 = 0.0, y64 = 0.0;
+  float x = 0.0f, y = 0.0f, th = 0.0f;
+  uint32_t r = 0;
+  if (act) {
+    if constexpr (P64) {
+      x64 = src.x64[j];
+      y64 = src.y64[j];
+      x = static_cast<float>(x64);
+      y = static_cast<float>(y64);
+    } else {
+      x = src.x[j];
+      y = src.y[j];
+    }
+    th = src.th[j];
+    r = rank[j];
+  }
+  uint32_t k = 0;
+  for (uint32_t ii = g.block_inst[blk];; ii++) {  // block-uniform walk
+    const Instance in = g.insts[ii];
+    const uint32_t end = in.agent_off + in.agent_count;
+    if (act && j >= in.agent_off && j < end)
+      k = key_of(x, y, th, in, g.params[ii], g.cell_log2, g.sort_key);
+    if (last < end || ii + 1u >= g.ninst) break;
+  }
+  if (!act) return;
+  const uint32_t d = offset[k] + r;
+  if (d >= g.total) return;  // unreachable: the count kernel's bins
+  if constexpr (P64) {
+    dst.x64[d] = x64;
+    dst.y64[d] = y64;
+  } else {
+    dst.x[d] = x;
+    dst.y[d] = y;
+  }
+  dst.th[d] = th;
+  dst.v[d] = src.v[j];
+  dst.id[d] = src.id[j];
 }
 
 __global__ __launch_bounds__(kAgentBlock) void canonical_copy_kernel(
@@ -508,9 +581,18 @@ void launch_morton_sort(const Pool& pool, const AgentSoA& src, const AgentSoA& d
   const SortArgs g{pool.inst,          pool.params,   pool.agent_block_inst, pool.count,
                    pool.total_agents,  pool.sort_cell_log2, pool.sort_key,   pool.xcd_remap};
   const uint32_t nb = blocks_for(pool.total_agents, kSortSlots);
-  count_kernel<<<nb, kAgentBlock, 0, stream>>>(g, src, pool.pos64, s.count);
+  if (s.rank)
+    count_kernel<true><<<nb, kAgentBlock, 0, stream>>>(g, src, pool.pos64, s.count, s.rank);
+  else
+    count_kernel<false><<<nb, kAgentBlock, 0, stream>>>(g, src, pool.pos64, s.count, nullptr);
   scan(s, s.count, pool.total_bins, s.offset, 0, stream);
-  if (pool.pos64)
+  if (s.rank) {
+    const uint32_t na = blocks_for(pool.total_agents, kAgentBlock);
+    if (pool.pos64)
+      scatter_ranked_kernel<true><<<na, kAgentBlock, 0, stream>>>(g, src, dst, s.rank, s.offset);
+    else
+      scatter_ranked_kernel<false><<<na, kAgentBlock, 0, stream>>>(g, src, dst, s.rank, s.offset);
+  } else if (pool.pos64)
     scatter_kernel<true><<<nb, kAgentBlock, 0, stream>>>(g, src, dst, s.count, s.offset);
   else
     scatter_kernel<false><<<nb, kAgentBlock, 0, stream>>>(g, src, dst, s.count, s.offset);
