@@ -1438,7 +1438,7 @@ class Engine {
     uint64_t units = 0, bins = 0;
     for (size_t k = 0; k < spec.size(); k++) {
       Instance& in = inst[k];
-      plan_trail(in, cfg.storage, cfg.trail_rows);
+      plan_trail(in, cfg.storage, cfg.trail_rows, total_cells);
       in.unit_off = static_cast<uint32_t>(units);
       units += in.units;
       uint32_t cl = cfg.sort_cell_log2;

@@ -280,8 +280,9 @@ inline uint64_t storage_bytes(int storage) { return storage == SLM_STORAGE_F32 ?
 inline uint32_t blocks_for(uint64_t n, uint32_t b) { return static_cast<uint32_t>((n + b - 1) / b); }
 
 // Host-side layout of one instance's trail pass: fills tile_rows, ntx, units.
-// rows > 0 fixes the tile height; 0 takes plan_trail's own choice.
-void plan_trail(Instance& in, int storage, uint32_t rows);
+// rows > 0 fixes the tile height; 0 takes plan_trail's own choice.  pool_cells: the
+// cells of all instances, which one launch covers.
+void plan_trail(Instance& in, int storage, uint32_t rows, uint64_t pool_cells);
 // Host-side layout of one instance's re-sort bins: fills nbins (clamped to
 // 2^31), nbx, nby, and returns the exact bin count.
 uint64_t plan_bins(Instance& in, uint32_t cell_log2);
