@@ -91,6 +91,7 @@ constexpr uint64_t kMaxPoolCells = 1ull << 40;
 constexpr uint64_t kMaxAgents = 0xffffff00ull;    // u32 slot index, whole blocks
 constexpr float kMaxSensorDistance = 4194304.0f;  // keeps sensor taps inside i32
 constexpr uint64_t kMaxTotalBins = 1ull << 30;
+constexpr uint64_t kMaxTrailUnits = 1ull << 26;   // waves of a launch, all below 2^32 threads
 constexpr float kMaxTrailValue = 0x1p100f;        // keeps every 3x3 window sum finite
 constexpr uint32_t kKnownFlags = SLM_FLAG_NO_XCD_REMAP | SLM_FLAG_F64_POSITIONS |
                                  SLM_FLAG_TILED_SENSING | SLM_FLAG_STOCHASTIC_ROUNDING |
@@ -1436,9 +1437,18 @@ class Engine {
     uint64_t total_cells = 0;
     for (size_t k = 0; k < spec.size(); k++) total_cells += cells(k);
     uint64_t units = 0, bins = 0;
+    // 4-row tiles and single cells of very many narrow rows can be more waves than one
+    // launch takes (2^32 threads): those pools take the tallest tiles
+    uint32_t rows = cfg.trail_rows;
+    for (Instance& in : inst) {
+      plan_trail(in, cfg.storage, rows, total_cells);
+      units += in.units;
+    }
+    if (rows == 0 && units >= kMaxTrailUnits) rows = 64;
+    units = 0;
     for (size_t k = 0; k < spec.size(); k++) {
       Instance& in = inst[k];
-      plan_trail(in, cfg.storage, cfg.trail_rows, total_cells);
+      plan_trail(in, cfg.storage, rows, total_cells);
       in.unit_off = static_cast<uint32_t>(units);
       units += in.units;
       uint32_t cl = cfg.sort_cell_log2;

@@ -38,3 +38,19 @@ def test_mixed_pools(slm, orc, storage, dims):
     orc.step(a1, t1, s, 3, storage=storage)
     assert_bitwise(ga, a1, "agents 1")
     assert_bitwise(out[0][1], t1, "trail 1")
+
+
+def test_more_rows_than_one_launch_of_short_tiles(slm):
+    """2^32 cells in rows of one strip: 4-row tiles would be 2^27 waves."""
+    w, h, count = 8, 1 << 23, 64
+    s = preset(slm, "Default")
+    specs = [slm.InstanceSpec(w, h, 200, seed=k, params=s) for k in range(count)]
+    with slm.Batch(specs, storage="bf16", graph_chunk=0) as b:
+        b.step(2)
+        got = {k: (b.read_agents(k), b.read_trail(k)) for k in (0, count - 1)}
+    for k, (a, t) in got.items():
+        print(f"[trail choice] instance {k} of {count}", flush=True)
+        with slm.Simulation(w, h, 200, seed=k, params=s, storage="bf16") as sim:
+            sim.step(2)
+            assert_bitwise(a, sim.read_agents(), f"agents {k}")
+            assert np.array_equal(t, sim.read_trail())
