@@ -341,7 +341,7 @@ struct RenderArgs {
   uint32_t tex_w, tex_h;
   float scale, off_x, off_y;
   uint32_t* out;      // tex_w * tex_h RGBA8 pixels, row-major
-  uint32_t rounds;    // set by launch_render: rounds of rows per workgroup
+  uint32_t rounds, lane_log2;  // set by launch_render: rounds of rows per workgroup, lanes per row
 };
 // Fills the fit fields of `a` as src/display.wgsl:48-72 computes them.
 void render_fit(uint32_t width, uint32_t height, uint32_t tex_w, uint32_t tex_h, RenderArgs& a);

@@ -542,31 +542,31 @@ __global__ void encode_trail_kernel(const float* in, uint64_t cells, void* t) {
 //
 // HBM-bound on large textures (a cell read and 4 bytes written per pixel), latency
 // on small ones.  A lane draws 4 pixels of a row (at scale 1 four neighbours, with
-// one load and one 16-byte store), a workgroup 256 pixels by kRenderRows rows per
-// round and a.rounds rounds, with the table merged into one word per entry in LDS.
+// one load and one 16-byte store), a row takes 2^a.lane_log2 lanes per 4 of its
+// pixels (64 from 129 columns on; fewer on narrow textures, so that a wave draws
+// several rows of them), and a workgroup draws a.rounds rounds of rows, with the table
+// merged into one word per entry in LDS.  The next round's cells are loaded before
+// the present one is drawn, the first before the table is there.
 // Against one pixel per lane, with a 64-bit division for its row and three byte
-// lookups, a picture of the grid's size takes 108 us instead of 226 (8192^2 f32;
-// 79 instead of 229 in bf16), 21 instead of 44 (4096^2 f32), 9.8 instead of 17.3
-// (3001 x 2003 bf16); the picture's store bounds the large ones.
-constexpr uint32_t kRenderCols = 256, kRenderRows = 4;
+// lookups, a picture of the grid's size takes 97 us instead of 229 (8192^2 f32;
+// 79 instead of 231 in bf16), 21 instead of 43 (4096^2 f32), 9.1 instead of 17
+// (3001 x 2003 bf16), 3.6 instead of 3.8 (256^2); the picture's store bounds the large
+// ones.  (With 64 lanes to every row 8 x 100000 took 14 us instead of 3.4; a row of 33
+// pixels still leaves lanes idle: 33 x 30000 4.8 us instead of 4.4.)
+constexpr uint32_t kRenderLanes = 256;
 
 template <int S, bool kDecode>
-__global__ __launch_bounds__(256) void render_kernel(RenderArgs a, LutBytes lut) {
+__global__ __launch_bounds__(kRenderLanes) void render_kernel(RenderArgs a, LutBytes lut) {
   using elem = typename Codec<S>::elem;
   __shared__ uint32_t s_rgba[256];
-  {
-    const uint32_t k = threadIdx.x;
-    auto byte = [&](uint32_t b) { return (lut.word[b >> 2] >> ((b & 3u) * 8u)) & 0xffu; };
-    s_rgba[k] = byte(k) | (byte(k + 256u) << 8) | (byte(k + 512u) << 16) | 0xff000000u;
-  }
-  __syncthreads();
-  // the lane's pixel columns: neighbours at scale 1, else 64 apart, so that a load's
-  // lanes read as close together as the scale allows
+  // the lane's pixel columns: neighbours at scale 1, else as far apart as the row has
+  // lanes, so that a load's lanes read as close together as the scale allows
   const bool unit = a.scale == 1.0f;
-  const uint32_t lane = threadIdx.x & 63u, step = unit ? 1u : 64u;
-  const uint32_t x0 = blockIdx.x * kRenderCols + (unit ? lane * 4u : lane);
-  if (x0 >= a.tex_w) return;
-  const uint32_t n = min(4u, (a.tex_w - x0 + step - 1u) / step);  // pixels of this lane
+  const uint32_t lanes = 1u << a.lane_log2, rows = kRenderLanes >> a.lane_log2;
+  const uint32_t lane = threadIdx.x & (lanes - 1u), step = unit ? 1u : lanes;
+  const uint32_t x0 = blockIdx.x * (4u * lanes) + (unit ? lane * 4u : lane);
+  // pixels of this lane
+  const uint32_t n = x0 < a.tex_w ? min(4u, (a.tex_w - x0 + step - 1u) / step) : 0u;
   // their cell columns, -1 outside the grid: the same for every row
   int col[4];
 #pragma unroll
@@ -577,30 +577,50 @@ __global__ __launch_bounds__(256) void render_kernel(RenderArgs a, LutBytes lut)
   }
   const bool run = unit && col[0] >= 0 && col[1] == col[0] + 1 && col[2] == col[0] + 2 &&
                    col[3] == col[0] + 3;  // 4 neighbouring cells
+  struct Cells {
+    elem v[4];
+    bool in;  // the row lies in the grid
+  };
+  auto fetch = [&](uint32_t py) {
+    Cells c{};
+    const float ry = static_cast<float>(py) - a.off_y;
+    const float fy = unit ? ry : ry / a.scale;
+    c.in = n != 0u && py < a.tex_h && fy >= 0.0f && fy < a.sim_h;
+    if (c.in) {
+      const elem* row = static_cast<const elem*>(a.trail) +
+                        static_cast<uint64_t>(static_cast<int>(fy)) * a.width;
+      if (run) {
+        __builtin_memcpy(c.v, row + col[0], sizeof c.v);
+      } else {
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+          if (col[k] >= 0) c.v[k] = row[col[k]];
+      }
+    }
+    return c;
+  };
+  uint32_t py = blockIdx.y * (rows * a.rounds) + (threadIdx.x >> a.lane_log2);
+  Cells next = fetch(py);
   const DevParams p = kDecode ? *a.decode : DevParams{};
+  {
+    const uint32_t k = threadIdx.x;
+    auto byte = [&](uint32_t b) { return (lut.word[b >> 2] >> ((b & 3u) * 8u)) & 0xffu; };
+    s_rgba[k] = byte(k) | (byte(k + 256u) << 8) | (byte(k + 512u) << 16) | 0xff000000u;
+  }
+  __syncthreads();
   auto colour = [&](uint32_t raw) {
     float t = kDecode ? deposit_decay<S>(raw, p) : Codec<S>::value(raw);
     t = t < 0.0f ? 0.0f : (t > 1.0f ? 1.0f : t);
     return s_rgba[static_cast<uint32_t>(t * 255.0f)];
   };
-  uint32_t py = blockIdx.y * (kRenderRows * a.rounds) + (threadIdx.x >> 6);
-  for (uint32_t r = 0; r < a.rounds && py < a.tex_h; r++, py += kRenderRows) {
-    const float ry = static_cast<float>(py) - a.off_y;
-    const float fy = unit ? ry : ry / a.scale;
+  for (uint32_t r = 0; r < a.rounds && py < a.tex_h; r++, py += rows) {
+    const Cells cell = next;
+    if (r + 1u < a.rounds) next = fetch(py + rows);
     uint32_t rgba[4] = {0xff000000u, 0xff000000u, 0xff000000u, 0xff000000u};
-    if (fy >= 0.0f && fy < a.sim_h) {
-      const elem* row = static_cast<const elem*>(a.trail) +
-                        static_cast<uint64_t>(static_cast<int>(fy)) * a.width;
-      if (run) {
-        elem cell[4];
-        __builtin_memcpy(cell, row + col[0], sizeof cell);
+    if (cell.in) {
 #pragma unroll
-        for (int k = 0; k < 4; k++) rgba[k] = colour(cell[k]);
-      } else {
-#pragma unroll
-        for (int k = 0; k < 4; k++)
-          if (col[k] >= 0) rgba[k] = colour(row[col[k]]);
-      }
+      for (int k = 0; k < 4; k++)
+        if (col[k] >= 0) rgba[k] = colour(cell.v[k]);
     }
     uint32_t* out = a.out + (static_cast<uint64_t>(py) * a.tex_w + x0);
     if (unit && n == 4u) {
@@ -1154,25 +1174,28 @@ void render_fit(uint32_t width, uint32_t height, uint32_t tex_w, uint32_t tex_h,
 void launch_render(const RenderArgs& args, const LutBytes& lut, int storage, hipStream_t stream) {
   if (args.tex_w == 0 || args.tex_h == 0) return;
   RenderArgs a = args;
-  const uint32_t gx = blocks_for(a.tex_w, kRenderCols);
+  a.lane_log2 = 6;
+  while (a.lane_log2 > 0 && (2u << a.lane_log2) >= a.tex_w) a.lane_log2--;
+  const uint32_t gx = blocks_for(a.tex_w, 4u << a.lane_log2);
+  const uint32_t rows = kRenderLanes >> a.lane_log2;
   // rounds per workgroup: up to 4 where 1024 workgroups remain (the table is then
   // merged for 4096 pixels), and at least as many as keep the grid's rows in range
   a.rounds = 4;
   while (a.rounds > 1 &&
-         static_cast<uint64_t>(gx) * blocks_for(a.tex_h, kRenderRows * a.rounds) < 1024u)
+         static_cast<uint64_t>(gx) * blocks_for(a.tex_h, rows * a.rounds) < 1024u)
     a.rounds >>= 1;
-  while (blocks_for(a.tex_h, kRenderRows * a.rounds) > 65535u) a.rounds <<= 1;
-  const dim3 grid(gx, blocks_for(a.tex_h, kRenderRows * a.rounds));
+  while (blocks_for(a.tex_h, rows * a.rounds) > 65535u) a.rounds <<= 1;
+  const dim3 grid(gx, blocks_for(a.tex_h, rows * a.rounds));
   const bool dec = a.decode != nullptr;
   if (storage == SLM_STORAGE_BF16)
-    dec ? render_kernel<SLM_STORAGE_BF16, true><<<grid, 256, 0, stream>>>(a, lut)
-        : render_kernel<SLM_STORAGE_BF16, false><<<grid, 256, 0, stream>>>(a, lut);
+    dec ? render_kernel<SLM_STORAGE_BF16, true><<<grid, kRenderLanes, 0, stream>>>(a, lut)
+        : render_kernel<SLM_STORAGE_BF16, false><<<grid, kRenderLanes, 0, stream>>>(a, lut);
   else if (storage == SLM_STORAGE_F16)
-    dec ? render_kernel<SLM_STORAGE_F16, true><<<grid, 256, 0, stream>>>(a, lut)
-        : render_kernel<SLM_STORAGE_F16, false><<<grid, 256, 0, stream>>>(a, lut);
+    dec ? render_kernel<SLM_STORAGE_F16, true><<<grid, kRenderLanes, 0, stream>>>(a, lut)
+        : render_kernel<SLM_STORAGE_F16, false><<<grid, kRenderLanes, 0, stream>>>(a, lut);
   else
-    dec ? render_kernel<SLM_STORAGE_F32, true><<<grid, 256, 0, stream>>>(a, lut)
-        : render_kernel<SLM_STORAGE_F32, false><<<grid, 256, 0, stream>>>(a, lut);
+    dec ? render_kernel<SLM_STORAGE_F32, true><<<grid, kRenderLanes, 0, stream>>>(a, lut)
+        : render_kernel<SLM_STORAGE_F32, false><<<grid, kRenderLanes, 0, stream>>>(a, lut);
 }
 
 void prime_persistent_trail() {
