@@ -924,8 +924,9 @@ class Engine {
     if (sort != sorting()) {
       uint64_t n = total_agents_;
       uint64_t pos = pos64() ? 16 : 8;
-      need += n * ((pos + 8 + (sort ? 4 : 0)) * (sort ? 2 : 1) + (sort ? 4 : 0));  // new arrays
-      need += n * (pos + 8);                                                      // snapshot
+      need += n * ((pos + 8 + (sort ? 4 : 0)) * (sort ? 2 : 1));              // new arrays
+      need += sort && n <= ranked_agents(pos64()) ? n * 4 : 0;                // and ranks
+      need += n * (pos + 8);                                                  // snapshot
     }
     size_t free_b = 0, total_b = 0;
     if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) {
