@@ -31,3 +31,14 @@ def test_narrow_textures(slm, orc, storage, w, h, textures):
         shown = display_point(orc, a, t, s, storage)
         tw, th = textures[1]
         assert_bitwise(sim.step_render(1, lut, tw, th), orc.render(shown, lut, tw, th), "display")
+
+
+def test_more_rows_than_a_launch_holds_groups(slm, orc):
+    """4 rows to a round: 65535 groups of 4 rounds end at row 1048560."""
+    w, h = 130, 1048577
+    lut = bytes(range(256)) * 3
+    with slm.Simulation(w, h, 100000, seed=3, params=preset(slm, "Default")) as sim:
+        sim.step(2)
+        t = sim.read_trail()
+        print(f"[render narrow] {w}x{h}", flush=True)
+        assert np.array_equal(sim.render(lut, w, h), orc.render(t, lut, w, h))
