@@ -1007,29 +1007,38 @@ void launch_gauss_t(const Pool& pool, const void* in, void* out, hipStream_t str
 
 }  // namespace
 
-// Whether rows take column strips.  A launch of strips takes
-// about 6.3 us + 0.48 ns a unit (7.3 us + 0.95 ns with 16-bit cells, whose unit is twice
-// as long), most of it one unit's latency; one of a cell per lane 4.7 us + 3.5 ns per
-// 1000 cells.  So strips win from 480000 (670000) cells of the launch on, and 34 cells
-// of the instance per strip cell column of a unit (34 v of its 256 v), which narrow
-// rows that leave most lanes idle do not have.  Strips / cells, us:
+// Whether rows take column strips, in tiles of `rows` rows (0: the library's choice, 4).
+// A launch of strips takes one unit's time, which grows with its rows, and some 0.1 ns
+// per row and unit (0.2 ns with 16-bit cells, whose unit is twice as long); one of a
+// cell per lane 4.7 us + 3.5 ns per 1000 cells.  So strips win from `few` cells of the
+// launch on, and 34 cells of the instance per cell column of a strip unit (34 v of its
+// 256 v), which narrow rows that leave most lanes idle do not have.  Strips of 4 rows /
+// cells, us:
 //   601 x 599 f32 6.7 / 6.4     801 x 799 f32 6.6 / 6.8     33 x 20001 f32 8.5 / 7.1
-//   801 x 799 bf16 7.8 / 7.3    1001 x 1003 bf16 7.6 / 8.7  63 x 20001 bf16 11.8 / 9.5
+//   801 x 799 bf16 7.8 / 7.3    1001 x 1003 bf16 7.8 / 8.7  63 x 20001 bf16 11.8 / 9.5
 //   10 of 1001 x 701 bf16 12.1 / 29.6   300 of 101 x 99 f32 11.0 / 14.7
-//   16384 of 16 x 16 bf16 67 / 28
-// Rows of whole strips keep them where their lanes are not mostly idle.
-static bool strips_pay(const Instance& in, uint32_t v, uint64_t pool_cells) {
+//   16384 of 16 x 16 bf16 67 / 26
+// and of 4, 8, 16, 32 and 64 rows at 2001 x 1003: f32 7.7, 8.8, 11.4, 20, 34 / 11.5, bf16
+// 7.9, 9.7, 13.6, 23, 40 / 12.2.
+// Rows of whole strips take them where their lanes are not mostly idle, and always in
+// tiles of a height that was asked for.
+static bool strips_pay(const Instance& in, uint32_t v, uint32_t rows, uint64_t pool_cells) {
+  if (in.width < v) return false;
+  const bool whole = in.width % v == 0u;
+  if (whole && rows) return true;
+  constexpr double kFew[2][5] = {{480e3, 1.0e6, 1.85e6, 5.0e6, 9.5e6},   // f32
+                                 {700e3, 1.3e6, 2.5e6, 5.5e6, 9.5e6}};  // 16-bit
+  const int log_rows = rows ? __builtin_ctz(rows) : 2;
+  const double few = whole ? 0.0 : kFew[v == 4u ? 0 : 1][log_rows - 2];
   const double cells = static_cast<double>(in.width) * in.height;
   const double units = static_cast<double>((in.width + 64u * v - 1u) / (64u * v)) *
                        ((in.height + 3u) / 4u);
-  const double few = in.width % v == 0u ? 0.0 : v == 4u ? 480e3 : 670e3;
   return cells - 34.0 * v * units >= few * cells / static_cast<double>(pool_cells);
 }
 
 void plan_trail(Instance& in, int storage, uint32_t fixed_rows, uint64_t pool_cells) {
   uint32_t v = storage == SLM_STORAGE_F32 ? 4u : 8u;
-  // a tile height that was asked for means strips
-  if (in.width >= v && (fixed_rows || strips_pay(in, v, pool_cells))) {
+  if (strips_pay(in, v, fixed_rows, pool_cells)) {
     in.ntx = (in.width + 64u * v - 1u) / (64u * v);
     // Rows per strip unit: fixed, or 4.  The shortest tiles are loaded whole, keep the
     // most waves, and their halo rows are found in the L2: at every size they take

@@ -40,6 +40,35 @@ def test_mixed_pools(slm, orc, storage, dims):
     assert_bitwise(out[0][1], t1, "trail 1")
 
 
+# odd row lengths around whole strips, and whole waves of them, that a launch of many
+# cells takes in strips (a row must have more than 34 cells in f32, 68 in 16 bits)
+ODD = {"f32": [63, 65, 129, 255, 257, 259, 261, 511, 513, 1021], "16": [127, 129, 255, 511, 513, 517, 519, 521, 1025]}
+
+
+@pytest.mark.parametrize("storage", ["f32", "bf16", "bf16sr", "f16"])
+@pytest.mark.parametrize("rows,streaming", [(0, 0), (4, 3), (8, 0), (16, 3), (64, 1)])
+def test_small_odd_grids_in_a_large_launch(slm, orc, storage, rows, streaming):
+    s = preset(slm, "Default")
+    kind = "bf16" if storage == "bf16sr" else storage
+    widths = ODD["f32" if storage == "f32" else "16"]
+    dims = [(w, (1, 2, 3, 5, 17, 67)[k % 6]) for k, w in enumerate(widths)]
+    specs = [slm.InstanceSpec(w, h, 200, seed=k, params=s) for k, (w, h) in enumerate(dims)]
+    specs.append(slm.InstanceSpec(8192, 4096, 0, seed=99, params=s))  # 33 million cells
+    rng = np.random.default_rng(rows * 8 + streaming)
+    print(f"[trail choice] odd grids {storage} rows={rows} streaming={streaming}", flush=True)
+    with slm.Batch(specs, storage=kind, stochastic_rounding=storage == "bf16sr") as b:
+        b.set_tuning(trail_rows=rows, streaming=streaming)
+        state = []
+        for k, (w, h) in enumerate(dims):
+            b.write_trail(k, rng.uniform(0, 1, (h, w)).astype(np.float32))
+            state.append((b.read_agents(k), b.read_trail(k)))
+        b.step(3)
+        for k, ((w, h), (a, t)) in enumerate(zip(dims, state)):
+            orc.step(a, t, s, 3, storage=storage)
+            assert_bitwise(b.read_trail(k), t, f"trail {w}x{h}")
+            assert_bitwise(b.read_agents(k), a, f"agents {w}x{h}")
+
+
 def test_more_rows_than_one_launch_of_short_tiles(slm):
     """2^32 cells in rows of one strip: 4-row tiles would be 2^27 waves."""
     w, h, count = 8, 1 << 23, 64
