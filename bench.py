@@ -20,7 +20,9 @@ The plain leg runs a fixed launch tuning (flags; by default 16-row trail
 tiles, a re-sort every 15 steps into 8x8-cell bins, 1024 agents per agent-pass
 workgroup and non-temporal trail-pass loads and stores; the library's
 autotuner found the bins, and sweeps over 20, 300 and 2000 steps chose the
-interval, the workgroup size and the streaming mode).
+interval, the workgroup size and the streaming mode).  Its agents sense through
+tile windows, by the library's choice, where these fit; --global-sensing turns
+them off.
 Before its warmup the batched (or combined) leg lets the library's autotuner
 choose its tuning (re-sort interval and bin size, agents per workgroup, trail
 tile rows, tiled sensing, instance groups, streaming) on its own
@@ -63,15 +65,14 @@ WRITE_SIZE_SCALE = 1.0
 # the dispatches of the timed steps, scaled as above) for exactly the run a
 # line describes: keyed by the workload, the launch tuning (re-sort interval,
 # bin log2, trail rows, agents per group, streaming, re-sort key) and the timed and warmup
-# step counts.  A line whose run has no entry reports traffic null.  Sources:
-# profiles/agents_kernel_plain_traffic.md (20 timed steps after 5 warmup, and
-# 2000 after 100).
+# step counts.  A line whose run has no entry reports traffic null.  Source:
+# profiles/tile_windows_counters.md (20 timed steps after 5 warmup, and 2000 after 100).
 MEASURED_TRAFFIC = {
     # (kernel, W, H, N, storage, tuning, steps, warmup): (FETCH KiB, WRITE KiB)
-    ("agents_kernel", 4096, 4096, 1 << 24, "f32", (15, 3, 16, 1024, 3, 0), 20, 5):
-        (181524, 278540),
-    ("agents_kernel", 4096, 4096, 1 << 24, "f32", (15, 3, 16, 1024, 3, 0), 2000, 100):
-        (169235, 219605),
+    ("agents_tiled_kernel", 4096, 4096, 1 << 24, "f32", (15, 3, 16, 1024, 3, 0), 20, 5):
+        (187655, 286671),
+    ("agents_tiled_kernel", 4096, 4096, 1 << 24, "f32", (15, 3, 16, 1024, 3, 0), 2000, 100):
+        (182780, 221504),
 }
 
 
@@ -88,6 +89,12 @@ def measured_traffic(kernel, args):
 def agent_bytes(sb, pos64=False):
     # 16 B state read + 16 B state write + 12 sensor taps + deposit read and write
     return 32 + 14 * sb + (16 if pos64 else 0)
+
+
+def tiled_agent_bytes(sb, cells, agents, pos64=False):
+    # 16 B state read + 16 B state write + each cell read once + a deposit written per
+    # agent at most (the windows' overlaps and the marks of shared cells are not counted)
+    return 32 + sb * cells / agents + sb + (16 if pos64 else 0)
 
 
 def trail_bytes(sb):
@@ -121,6 +128,9 @@ def parse():
                          "classes log2 in bits 0-2, 0x10 = bin at the centre sensor)")
     ap.add_argument("--tiled", action="store_true",
                     help="plain leg: LDS-staged sensing from per-tile work lists")
+    ap.add_argument("--global-sensing", action="store_true",
+                    help="plain leg: sensing from global memory, where the library would choose "
+                         "tile windows")
     ap.add_argument("--window", action="store_true",
                     help="plain leg: LDS-staged sensing through per-workgroup windows")
     ap.add_argument("--batch-tuning", default="",
@@ -241,6 +251,10 @@ LIMITER = {
                       "waits on the L1 59%; profiles/agents_kernel_l1_counters.md), then VALU; "
                       "DRAM traffic is well below the algorithmic bytes because the taps hit L2, "
                       "so the kernel is not HBM-bound"),
+    "agents_tiled_kernel": ("VALU issue, 46 to 88% of its cycles (557 instructions a wave of two "
+                            "agents a lane, at 2.3 to 4.4 cycles), beside the vector L1 (36%) and "
+                            "the LDS (29%); profiles/tile_windows_counters.md.  Steps whose windows "
+                            "do not fit run agents_kernel and are part of the mean"),
     "trail_kernel": "HBM bandwidth",
 }
 
@@ -274,6 +288,8 @@ def plain_leg(slm, args):
                              stochastic_rounding=plain_sr(args))
         sim.set_tuning(trail_rows=args.trail_rows, agents_per_group=args.agents_per_group,
                        streaming=args.streaming, sort_key=args.sort_key)
+        if args.global_sensing:
+            sim.set_tuning(tiled_sensing=slm.SENSING_GLOBAL)
         return sim
 
     sim = make()
@@ -301,6 +317,7 @@ def plain_leg(slm, args):
     rep = make()
     if tuning.get("autotuned"):
         rep.set_tuning(**{f: tuning[f] for f in TUNING_FIELDS})
+    tiled = rep.sensing() == 1  # the first step re-sorts
     rep.step(args.warmup)
     rep.synchronize()
     t0 = time.perf_counter()
@@ -309,11 +326,13 @@ def plain_leg(slm, args):
     rep.close()
     log(f"plain: the same {K} steps again with per-kernel events in {m_elapsed:.3f} s")
     a_bytes, t_bytes = agent_bytes(sb, args.f64_positions) * N, trail_bytes(sb) * W * H
+    if tiled:
+        a_bytes = round(tiled_agent_bytes(sb, W * H, N, args.f64_positions) * N)
     return {
         "value": N * K / elapsed, "elapsed": elapsed, "steps": K, "segments": seg,
         "measure_value": N * K / m_elapsed,
         "agents_s": a_s, "trail_s": t_s, "sort_s": s_s, "mass": mass,
-        "agents_roof": roofline("agents_kernel", a_bytes, a_s),
+        "agents_roof": roofline("agents_tiled_kernel" if tiled else "agents_kernel", a_bytes, a_s),
         "trail_roof": roofline("trail_kernel", t_bytes, t_s),
         "cells": W * H, "agents": N, "state0": state0, "presets": presets, "tuning": tuning,
     }
@@ -546,7 +565,7 @@ def main():
         dram = traffic / (dominant["avg_launch_us"] * 1e-6) / 1e9
         dominant["dram_gbps"] = round(dram, 1)
         dominant["dram_frac"] = round(dram / HBM_PEAK_GBPS, 4)
-        dominant["traffic_source"] = "profiles/agents_kernel_plain_traffic.md (same command)"
+        dominant["traffic_source"] = "profiles/tile_windows_counters.md (same command)"
     graph_steps, eager_steps = graph_split(plain["segments"], args.graph_chunk)
     out = {
         "metric": METRIC,
@@ -589,6 +608,7 @@ def main():
                      if plain["trail_roof"]["bytes_per_launch"] <= 256e6 else ""),
         },
         "agents_kernel": {
+            "kernel": plain["agents_roof"]["kernel"],
             "avg_launch_us": plain["agents_roof"]["avg_launch_us"],
             "achieved_gbps": plain["agents_roof"]["achieved"],
             "agent_updates_per_s": N / plain["agents_s"],

@@ -667,7 +667,9 @@ __global__ __launch_bounds__(kAgentBlock) void agents_kernel(
 // the work list or the time since the re-sort) and angles and parameters are in
 // the ordinary range, else it takes agent_update and reads global memory.
 //
-// The update itself is then bound by VALU issue.  On gfx950 f32 multiply, add
+// The update itself is then mostly VALU issue: 557 instructions a wave of two agents a
+// lane take 46 to 88% of the pass's cycles, the L1 36%, the LDS 29% (4096^2 f32, 2^24
+// agents, trails formed).  On gfx950 f32 multiply, add
 // and fma, and/xor/bitop3, right shifts and 32-bit adds issue in 2.3 cycles per
 // wave when every operand is a vector register or a literal; with a scalar
 // register operand, and for compares, selects, conversions, rounding, left
