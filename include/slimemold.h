@@ -163,7 +163,8 @@ typedef struct slm_info {
   int32_t storage;
   int32_t device;
   uint64_t steps_done;
-  uint64_t device_bytes; /* device memory held by the handle */
+  uint64_t device_bytes; /* device memory held by the handle, the buffer (up to 16 MiB)
+                            that it keeps for copies to and from the host included */
   uint32_t resort_interval, graph_chunk;
 } slm_info;
 

@@ -1239,10 +1239,11 @@ class Engine {
   }
 
   // The device buffer that copies to and from the host go through, kept between
-  // calls up to kStagingKept bytes (a larger one is freed when its call ends; not
-  // counted in device_bytes).  Allocating and freeing it on each call, and copying the
+  // calls up to kStagingKept bytes (a larger one is freed when its call ends).
+  // Allocating and freeing it on each call, and copying the
   // trail to be written for its -0 cells, took 1.2 of the 2.6 ms of writing, stepping
-  // and reading 1001 x 701 cells with 3 * 10^5 agents.  A call uses it from reserve until the
+  // and reading 1001 x 701 cells with 3 * 10^5 agents (a handle's first such pass still
+  // allocates it: 1.63 ms before, 1.30 now).  A call uses it from reserve until the
   // stream has been waited for, and a handle is used by one thread at a time.
   static constexpr size_t kStagingKept = size_t(16) << 20;
   struct Staging {
@@ -1272,6 +1273,12 @@ class Engine {
   };
   void* staging_ = nullptr;
   size_t staging_bytes_ = 0;
+
+ public:
+  // Device memory of the handle: its buffers and the kept staging buffer.
+  uint64_t held_bytes() const { return device_bytes + staging_bytes_; }
+
+ private:
   void free_staging() {
     if (staging_) (void)hipFree(staging_);
     staging_ = nullptr;
@@ -2460,7 +2467,7 @@ int slm_get_info(const slm_sim* s, slm_info* out) {
   out->storage = e.cfg.storage;
   out->device = e.cfg.device;
   out->steps_done = e.steps_done;
-  out->device_bytes = e.device_bytes;
+  out->device_bytes = e.held_bytes();
   out->resort_interval = e.cfg.resort_interval;
   out->graph_chunk = e.cfg.graph_chunk;
   return SLM_OK;
@@ -2903,7 +2910,7 @@ int slm_batch_get_info(const slm_batch* b, slm_batch_info* out) {
     out->total_cells += e.cells(k);
   }
   out->steps_done = e.steps_done;
-  out->device_bytes = e.device_bytes;
+  out->device_bytes = e.held_bytes();
   return SLM_OK;
   SLM_ENTRY_END
 }
