@@ -361,7 +361,10 @@ void launch_unpack_positions64(const Instance& in, const AgentSoA& a, const doub
 // 2^14 agents on 256^2 16.3 / 19.6, 2^18 on 1024^2 22.9 / 25.1, 2^21 on 2048^2 41.7 /
 // 44.9, 2^22 on 256^2 57.5 / 60.5, 2048^2 61.9 / 66.0, 4096^2 78 / 71, 2^23 on 2048^2
 // 126 / 116; with f64 positions 2^20 on 1024^2 34.4 / 34.5, 2^22 89 / 79.
-constexpr uint64_t ranked_agents(bool pos64) { return pos64 ? 1u << 21 : 1u << 22; }
+// Beside other work on the GPU the LDS form does better, whose stores take less of the
+// L1: three simulations of 2048^2 with 2^22 agents and long sensors, each on its stream,
+// take 1139 us per 10 steps and picture instead of 1149.
+constexpr uint64_t ranked_agents(bool pos64) { return pos64 ? 1u << 21 : 3u << 20; }
 struct SortScratch {
   uint32_t* rank;      // per slot: rank inside its bin; nullptr beyond ranked_agents
   uint32_t* count;     // per bin: agents, then (no rank) those still to be scattered

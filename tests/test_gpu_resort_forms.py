@@ -1,4 +1,4 @@
-"""Both forms of the re-sort, on either side of the agent count that parts them (2^22,
+"""Both forms of the re-sort, on either side of the agent count that parts them (3 * 2^20,
 2^21 with f64 positions): agents in any order, crowds in bins that share a table entry,
 and neighbouring instances whose agents wrap into each other's bins, equal the run that
 is never re-sorted."""
@@ -10,7 +10,7 @@ from parity_util import assert_bitwise, preset
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("n,f64", [(1 << 22, False), ((1 << 22) + 1, False), (1 << 21, True),
+@pytest.mark.parametrize("n,f64", [(3 << 20, False), ((3 << 20) + 1, False), (1 << 21, True),
                                    ((1 << 21) + 1023, True)])
 @pytest.mark.parametrize("key", [0, 3])
 def test_crowds_and_strays(slm, n, f64, key):
@@ -36,7 +36,7 @@ def test_crowds_and_strays(slm, n, f64, key):
     assert_bitwise(out[1][1], out[0][1], "trail")
 
 
-@pytest.mark.parametrize("count,agents,f64", [(40, 6001, False), (750, 6001, False),
+@pytest.mark.parametrize("count,agents,f64", [(40, 6001, False), (530, 6001, False),
                                               (360, 6001, True)])
 def test_instances_of_many_bins(slm, count, agents, f64):
     specs = [slm.InstanceSpec(40, 300, agents, seed=k, params=preset(slm, "Waves"))
