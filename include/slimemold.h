@@ -117,7 +117,7 @@ typedef struct slm_config {
  * sensor reach plus drift since the re-sort) in LDS and sense from there; agents
  * that the window does not cover, and tiles whose window does not fit 80 KiB, read
  * global memory, so results are unchanged.  Without the flag the library does so
- * by itself where it pays (from 2^21 agents on, 2^22 with f64 positions, some 1600
+ * by itself where it pays (from 2^21 agents on, 3 * 2^20 with f64 positions, some 1600
  * to a tile, windows that fit for a number of steps); with it, wherever there is a
  * re-sort. */
 #define SLM_FLAG_TILED_SENSING 0x4u

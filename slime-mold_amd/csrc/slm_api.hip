@@ -1588,7 +1588,7 @@ class Engine {
 
   // Whether the pool's agents sense through tile windows of the library's own
   // accord: with the plain re-sort key, one launch per pass over the pool and no
-  // other sensing asked for, from 2^21 agents on (2^22 with f64 positions, whose
+  // other sensing asked for, from 2^21 agents on (3 * 2^20 with f64 positions, whose
   // workgroups hold half the waves) and with enough of them to a tile.  Fewer agents
   // do not fill the chip with workgroups of whole tiles; tiles that hold few, or that
   // the grid's edge cuts to slivers (the mean is weighed by the share of the tiles'
@@ -1600,12 +1600,14 @@ class Engine {
   //     1975    82 of 160^2, 2^21 agents 1.03, 2^22 0.92 (f64 1.05 to 1.13, 0.96 to 1.04)
   //     2048    one 2048^2 0.86, 1024 of 64^2 0.91 (f64 0.85, 1.0)
   //     4096    one 2048^2 0.75, one 4096^2 0.68, 512 of 64^2 0.83
+  // and with f64 positions, over single grids from 1900 on: 2^21 agents 0.88 to 1.10,
+  // 2.8 * 10^6 0.93 to 1.07, 3.3 * 10^6 0.90 to 1.00, 2^22 0.82 to 0.96.
   bool auto_tiles() const {
     return !cfg.global_sensing && !(cfg.flags & SLM_FLAG_WINDOW_SENSING) &&
            windows_pay(cfg.resort_interval, cfg.instance_groups, cfg.sort_key);
   }
   bool windows_pay(uint32_t resort_interval, uint32_t instance_groups, uint32_t sort_key) const {
-    const uint64_t min_agents = pos64() ? 1u << 22 : 1u << 21;
+    const uint64_t min_agents = pos64() ? 3u << 20 : 1u << 21;
     const double min_per_tile = pos64() ? 1900.0 : 1550.0;
     constexpr double kTileCells = double(1u << (2 * kTileLog2));
     const double per_tile = static_cast<double>(total_agents_) / window_tiles_ *
