@@ -218,7 +218,7 @@ __device__ inline void store_row(void* dst, uint4 v, bool streaming) {
 // strip ends at the row's end and overlaps the one before it: both compute the
 // shared cells, to the same bits, and neither's halo is its neighbour's edge.
 // Against one cell per lane, with a division for its row and nine loads, such rows
-// take 11.4 us instead of 29 at 3001 x 2003 bf16, 131 instead of 295 at 8191^2 f32;
+// take 11.0 us instead of 29 at 3001 x 2003 bf16, 106 instead of 295 at 8191^2 f32;
 // the memory system serves the unaligned strips at about the aligned rate.
 struct StripColumns {
   uint32_t c, lcol, rcol;
@@ -545,14 +545,16 @@ __global__ void encode_trail_kernel(const float* in, uint64_t cells, void* t) {
 // one load and one 16-byte store), a row takes 2^a.lane_log2 lanes per 4 of its
 // pixels (64 from 129 columns on; fewer on narrow textures, so that a wave draws
 // several rows of them), and a workgroup draws a.rounds rounds of rows, with the table
-// merged into one word per entry in LDS.  The next round's cells are loaded before
-// the present one is drawn, the first before the table is there.
+// merged into one word per entry in LDS.  The first round's cells are loaded before the
+// table is there.  (With every round's loaded before the one before it is drawn, a step
+// with its picture takes 27.8 us instead of 27.0 at 2048^2 f16, 32.4 instead of 31.6 at
+// 3001 x 2003 bf16.)
 // Against one pixel per lane, with a 64-bit division for its row and three byte
-// lookups, a picture of the grid's size takes 97 us instead of 229 (8192^2 f32;
-// 79 instead of 231 in bf16), 21 instead of 43 (4096^2 f32), 9.1 instead of 17
-// (3001 x 2003 bf16), 3.6 instead of 3.8 (256^2); the picture's store bounds the large
+// lookups, a picture of the grid's size takes 103 us instead of 229 (8192^2 f32;
+// 72 instead of 231 in bf16), 21 instead of 43 (4096^2 f32), 8.7 instead of 17
+// (3001 x 2003 bf16), 4.3 instead of 5.4 (1600 x 900); the picture's store bounds the large
 // ones.  (With 64 lanes to every row 8 x 100000 took 14 us instead of 3.4; a row of 33
-// pixels still leaves lanes idle: 33 x 30000 4.8 us instead of 4.4.)
+// pixels still leaves lanes idle: 33 x 30000 4.8 us instead of 4.3.)
 constexpr uint32_t kRenderLanes = 256;
 
 template <int S, bool kDecode>
@@ -600,7 +602,7 @@ __global__ __launch_bounds__(kRenderLanes) void render_kernel(RenderArgs a, LutB
     return c;
   };
   uint32_t py = blockIdx.y * (rows * a.rounds) + (threadIdx.x >> a.lane_log2);
-  Cells next = fetch(py);
+  const Cells first = fetch(py);
   const DevParams p = kDecode ? *a.decode : DevParams{};
   {
     const uint32_t k = threadIdx.x;
@@ -614,10 +616,12 @@ __global__ __launch_bounds__(kRenderLanes) void render_kernel(RenderArgs a, LutB
     return s_rgba[static_cast<uint32_t>(t * 255.0f)];
   };
   for (uint32_t r = 0; r < a.rounds && py < a.tex_h; r++, py += rows) {
-    const Cells cell = next;
-    if (r + 1u < a.rounds) next = fetch(py + rows);
+    const Cells cell = r ? fetch(py) : first;
     uint32_t rgba[4] = {0xff000000u, 0xff000000u, 0xff000000u, 0xff000000u};
-    if (cell.in) {
+    if (cell.in && run) {
+#pragma unroll
+      for (int k = 0; k < 4; k++) rgba[k] = colour(cell.v[k]);
+    } else if (cell.in) {
 #pragma unroll
       for (int k = 0; k < 4; k++)
         if (col[k] >= 0) rgba[k] = colour(cell.v[k]);
@@ -1042,9 +1046,9 @@ void plan_trail(Instance& in, int storage, uint32_t fixed_rows, uint64_t pool_ce
     in.ntx = (in.width + 64u * v - 1u) / (64u * v);
     // Rows per strip unit: fixed, or 4.  The shortest tiles are loaded whole, keep the
     // most waves, and their halo rows are found in the L2: at every size they take
-    // the least time, or within 2% of it, in us, 4 / 8 / 16 / 64 rows:
-    //   1024^2 f32 7.0 / 8.4 / 11.2 / 36    4096^2 f32 21.8 / 23.0 / 23.1 / 41
-    //   8192^2 f32 102 / 107 / 107 / 118    8192^2 bf16 46.8 / 45.9 / 51.9 / 55.5
+    // the least time, or within 5% of it, in us, 4 / 8 / 16 / 64 rows:
+    //   1024^2 f32 6.8 / 8.2 / 10.7 / 34    4096^2 f32 21.4 / 22.7 / 23.0 / 40
+    //   8192^2 f32 99 / 105 / 106 / 116     8192^2 bf16 45.1 / 42.9 / 48.6 / 51.5
     // (taller tiles on larger grids, for at least 8192 waves, gave the last a 64-row
     // tile in f32 and a 16-row one in bf16)
     const uint32_t rows = fixed_rows ? fixed_rows : 4u;
